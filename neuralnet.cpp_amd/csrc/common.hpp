@@ -293,7 +293,8 @@ hipError_t launch_glu_interleave(hipStream_t st, const uint32_t* wq, const float
 // kscale (nullable, per k) multiplies the activations first (the transposed product's tau);
 // tau (nullable) is the per-row output factor.
 hipError_t launch_digits(hipStream_t st, const void* B, bool b16, const float* kscale, size_t K, size_t M, int8_t* xi,
-                         int32_t* rowsum, int32_t* ex);
+                         int32_t* rowsum, int32_t* ex, uint32_t* part);
+size_t digit_part_bytes(size_t M);  // part: pieces of the tokens' absmax
 hipError_t launch_digit_combine(hipStream_t st, const float* Yp, const float* tau, const int32_t* ex,
                                 const uint32_t* rp, const void* B, bool b16, const float* kscale, size_t N, size_t K,
                                 size_t M, void* Y, bool y16);

@@ -143,6 +143,141 @@ __global__ __launch_bounds__(kDigThreads) void k_digits(const void* __restrict__
     if (tid == 0) ex[m] = bad ? kSpecialToken : E;
 }
 
+// The digits of many tokens (M > 4) in two launches that read B along tokens, 64 at a time, so
+// that every load is one 256-byte row piece (k_digits' blocks each read one column of B, a line
+// per element: 71 us at K=2560, 220 us at K=6912 for 2048 tokens). The row count per block is
+// what lets a few tokens fill the chip too: the absmax of a token is taken in kDigParts pieces.
+//
+// k_digit_absmax: block (64 tokens, piece c of K): the largest |x| bit pattern of each token over
+// the piece, into part[c][m]. Compared as integers, infinities and NaN rank above every finite
+// value, so the flag of a special token needs no register of its own. Piece 0 also clears the
+// digit row sums that k_digit_rows adds to.
+// k_digit_rows: block (64 tokens, 128 columns): each wave makes the digits of 32 columns, lane =
+// token, then the block writes its 256 digit rows x 128 bytes as whole lines through LDS.
+// Bound by HBM: 4KM bytes read twice (the second time mostly from the memory-side cache) and
+// 4M Kp written. For 2048 f32 tokens (rocprofv3, absmax + rows): 6.0 + 9.7 us at K=2560, 13.4 +
+// 26.0 us at K=6912 with kscale (57 MB read, 57 MB written: 4.4 TB/s in the second kernel).
+constexpr int kDigTok = 64;        // tokens per block
+constexpr int kDigParts = 32;      // pieces of K for the absmax
+constexpr int kDigMaxThreads = 512;
+constexpr int kDigRowThreads = 256;
+constexpr int kDigCols = 128;      // columns per block of k_digit_rows (Kp is a multiple)
+
+// element type and kscale as template arguments: a uniform branch at each load would take the
+// loads out of flight one by one
+template <typename BT, bool KS>
+__device__ __forceinline__ float load_bt(const void* B, const float* kscale, int k, int M, int m)
+{
+    const float x = (float)reinterpret_cast<const BT*>(B)[(size_t)k * M + m];
+    return KS ? __fmul_rn(kscale[k], x) : x;
+}
+
+template <typename BT, bool KS>
+__global__ __launch_bounds__(kDigMaxThreads) void k_digit_absmax(const void* __restrict__ B,
+                                                                 const float* __restrict__ kscale, int K, int M,
+                                                                 int rows, uint32_t* __restrict__ part,
+                                                                 int32_t* __restrict__ rowsum)
+{
+    constexpr int NW = kDigMaxThreads / kWave;
+    constexpr int U = 14;  // loads in flight per lane
+    __shared__ uint32_t smax[NW][kDigTok];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int m = blockIdx.x * kDigTok + lane, c = blockIdx.y;
+    const int k1 = min(K, (c + 1) * rows);
+    const int ml = min(m, M - 1);  // loads past the ends repeat the last token or row
+    uint32_t mx = 0;
+    for (int k0 = c * rows + w; k0 < k1; k0 += NW * U)
+    {
+        float v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = load_bt<BT, KS>(B, kscale, min(k0 + u * NW, k1 - 1), M, ml);
+#pragma unroll
+        for (int u = 0; u < U; ++u) mx = max(mx, __builtin_bit_cast(uint32_t, v[u]) & 0x7FFFFFFFu);
+    }
+    smax[w][lane] = mx;
+    __syncthreads();
+    if (w != 0 || m >= M) return;
+#pragma unroll
+    for (int i = 1; i < NW; ++i) mx = max(mx, smax[i][lane]);
+    part[(size_t)c * M + m] = mx;
+    if (c == 0)
+#pragma unroll
+        for (int p = 0; p < 4; ++p) rowsum[4 * m + p] = 0;
+}
+
+template <typename BT, bool KS>
+__global__ __launch_bounds__(kDigRowThreads) void k_digit_rows(const void* __restrict__ B,
+                                                               const float* __restrict__ kscale, int K, int M, int Kp,
+                                                               const uint32_t* __restrict__ part, int parts,
+                                                               int8_t* __restrict__ xi, int32_t* __restrict__ rowsum,
+                                                               int32_t* __restrict__ ex)
+{
+    constexpr int NW = kDigRowThreads / kWave, KW = kDigCols / NW;  // columns per wave
+    // token t's four digit rows of the block's columns, 32 words each; one word more per token, so
+    // that the 64 lanes (tokens) of a word store fall on 64 banks
+    constexpr int ROWW = kDigCols / 4, TOKW = 4 * ROWW + 1;
+    __shared__ uint32_t dig[kDigTok * TOKW];
+    __shared__ int ssum[NW][4][kDigTok];
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int m0 = blockIdx.x * kDigTok, m = m0 + lane;
+    const int kb = blockIdx.y * kDigCols, kw = kb + w * KW;
+    const int ml = min(m, M - 1);  // loads past the ends repeat the last token or column
+    float v[KW];
+#pragma unroll
+    for (int i = 0; i < KW; ++i) v[i] = load_bt<BT, KS>(B, kscale, min(kw + i, K - 1), M, ml);
+    uint32_t mx = 0, pm[kDigParts];
+#pragma unroll
+    for (int c = 0; c < kDigParts; ++c) pm[c] = part[(size_t)min(c, parts - 1) * M + ml];
+#pragma unroll
+    for (int c = 0; c < kDigParts; ++c) mx = max(mx, pm[c]);
+    const bool bad = mx >= 0x7F800000u;  // an infinity or a NaN: all digits 0
+    int E = 0;
+    if (!bad) (void)frexpf(__builtin_bit_cast(float, mx), &E);  // |x| < 2^E (E = 0 for a zero token)
+    if (blockIdx.y == 0 && w == 0 && m < M) ex[m] = bad ? kSpecialToken : E;
+    const int shift = 30 - E;
+    int s[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < KW; i += 4)
+    {
+        // the four digits of X in one word: adding 128 to each of the low three bytes with carries
+        // and flipping their top bits back leaves byte p = d_p
+        uint32_t D[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+        {
+            const int X = (int)__builtin_rintf(ldexpf(bad || kw + i + j >= K ? 0.0f : v[i + j], shift));
+            D[j] = ((uint32_t)X + 0x00808080u) ^ 0x00808080u;
+        }
+        // 4 x 4 byte transpose: word p = digit p of the four columns
+        const uint32_t lo0 = __builtin_amdgcn_perm(D[1], D[0], 0x05010400u), lo1 = __builtin_amdgcn_perm(D[3], D[2], 0x05010400u);
+        const uint32_t hi0 = __builtin_amdgcn_perm(D[1], D[0], 0x07030602u), hi1 = __builtin_amdgcn_perm(D[3], D[2], 0x07030602u);
+        const uint32_t d[4] = {__builtin_amdgcn_perm(lo1, lo0, 0x05040100u), __builtin_amdgcn_perm(lo1, lo0, 0x07060302u),
+                               __builtin_amdgcn_perm(hi1, hi0, 0x05040100u), __builtin_amdgcn_perm(hi1, hi0, 0x07060302u)};
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+        {
+            dig[lane * TOKW + p * ROWW + (w * KW + i) / 4] = d[p];
+            s[p] = __builtin_amdgcn_sdot4((int)d[p], 0x01010101, s[p], false);
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < 4; ++p) ssum[w][p][lane] = s[p];
+    __syncthreads();
+    // 16-byte units: 8 lanes per digit row of the block (128 contiguous bytes of xi)
+#pragma unroll
+    for (int u0 = 0; u0 < kDigTok * 4 * (kDigCols / 16); u0 += kDigRowThreads)
+    {
+        const int u = u0 + tid, r = u / (kDigCols / 16), q = u % (kDigCols / 16);
+        const uint32_t* src = dig + (r >> 2) * TOKW + (r & 3) * ROWW + 4 * q;
+        const u32x4 x = {src[0], src[1], src[2], src[3]};
+        if (m0 + (r >> 2) < M)
+            *reinterpret_cast<u32x4*>(xi + (size_t)(4 * m0 + r) * Kp + kb + 16 * q) = x;
+    }
+    const int p = w;  // one digit per wave
+    if (m < M)
+        atomicAdd(&rowsum[4 * m + p], ssum[0][p][lane] + ssum[1][p][lane] + ssum[2][p][lane] + ssum[3][p][lane]);
+}
+
 // The same digits for a few long tokens (the split-k path, M <= 4): block (c, m) takes columns
 // [c * kChunk, (c + 1) * kChunk) of token m. Each block first reduces the absmax and the
 // non-finite flag over the whole token (every chunk of a token sees the same E, so the digits are
@@ -618,12 +753,47 @@ hipError_t launch_dg_m(hipStream_t st, const DigitGemvArgs& a, int M)
 
 }  // namespace
 
-hipError_t launch_digits(hipStream_t st, const void* B, bool b16, const float* kscale, size_t K, size_t M, int8_t* xi,
-                         int32_t* rowsum, int32_t* ex)
+namespace
+{
+
+template <typename BT, bool KS>
+hipError_t launch_digits_tok(hipStream_t st, const void* B, const float* kscale, size_t K, size_t M, int8_t* xi,
+                             int32_t* rowsum, int32_t* ex, uint32_t* part)
 {
     const size_t Kp = round_up(K, kTileK);
-    k_digits<<<dim3((unsigned)M), kDigThreads, 0, st>>>(B, b16, kscale, (int)K, (int)M, (int)Kp, xi, rowsum, ex);
+    const unsigned tiles = (unsigned)ceil_div(M, (size_t)kDigTok);
+    const size_t rows = ceil_div(K, (size_t)kDigParts), parts = ceil_div(K, rows);
+    hipLaunchKernelGGL((k_digit_absmax<BT, KS>), dim3(tiles, (unsigned)parts), dim3(kDigMaxThreads), 0, st, B, kscale,
+                       (int)K, (int)M, (int)rows, part, rowsum);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((k_digit_rows<BT, KS>), dim3(tiles, (unsigned)(Kp / kDigCols)), dim3(kDigRowThreads), 0, st, B,
+                       kscale, (int)K, (int)M, (int)Kp, part, (int)parts, xi, rowsum, ex);
     return hipGetLastError();
+}
+
+}  // namespace
+
+size_t digit_part_bytes(size_t M) { return (size_t)kDigParts * M * 4; }
+
+hipError_t launch_digits(hipStream_t st, const void* B, bool b16, const float* kscale, size_t K, size_t M, int8_t* xi,
+                         int32_t* rowsum, int32_t* ex, uint32_t* part)
+{
+    const size_t Kp = round_up(K, kTileK);
+    // one launch, one block per token, while the column reads stay few: a lone call of the two
+    // launches takes 1-2 us longer there (K=2560, whole product: M=40 23.4 against 24.6 us, M=256
+    // 44.5 against 42.1; K=1000, M=256 15.5 against 16.6; K=6912: M=5 26.0 against 28.1, M=8 29.4
+    // against 28.3)
+    if (M <= 6 || (K <= 4096 && K * M <= (size_t(1) << 18)))
+    {
+        k_digits<<<dim3((unsigned)M), kDigThreads, 0, st>>>(B, b16, kscale, (int)K, (int)M, (int)Kp, xi, rowsum, ex);
+        return hipGetLastError();
+    }
+    if (b16)
+        return kscale ? launch_digits_tok<_Float16, true>(st, B, kscale, K, M, xi, rowsum, ex, part)
+                      : launch_digits_tok<_Float16, false>(st, B, kscale, K, M, xi, rowsum, ex, part);
+    return kscale ? launch_digits_tok<float, true>(st, B, kscale, K, M, xi, rowsum, ex, part)
+                  : launch_digits_tok<float, false>(st, B, kscale, K, M, xi, rowsum, ex, part);
 }
 
 size_t digit_chunks(size_t K) { return ceil_div(round_up(K, kTileK), (size_t)kChunk); }

@@ -919,8 +919,8 @@ static nnhip_status matmul_digits(nnhip_ctx* ctx, const char* fn, const void* rp
         return NNHIP_OK;
     }
     const size_t b_xi = round_up(M4 * Kp, 256), b_rs = round_up(M4 * 4, 256), b_ex = round_up(M * 4, 256);
-    const size_t b_yp = N * M4 * 4;
-    st = ensure_ws(ctx, b_xi + b_rs + b_ex + b_yp, fn);
+    const size_t b_yp = round_up(N * M4 * 4, 256), b_part = digit_part_bytes(M);
+    st = ensure_ws(ctx, b_xi + b_rs + b_ex + b_yp + b_part, fn);
     if (st != NNHIP_OK) return st;
     const size_t ones = N > M4 ? N : M4;
     if (ctx->ones_words < ones)
@@ -935,7 +935,8 @@ static nnhip_status matmul_digits(nnhip_ctx* ctx, const char* fn, const void* rp
     int32_t* rs = reinterpret_cast<int32_t*>(w + b_xi);
     int32_t* ex = reinterpret_cast<int32_t*>(w + b_xi + b_rs);
     float* yp = reinterpret_cast<float*>(w + b_xi + b_rs + b_ex);
-    NNHIP_LAUNCH(fn, launch_digits(ctx->stream, B, b_f16 != 0, kscale, K, M, xi, rs, ex));
+    uint32_t* part = reinterpret_cast<uint32_t*>(w + b_xi + b_rs + b_ex + b_yp);
+    NNHIP_LAUNCH(fn, launch_digits(ctx->stream, B, b_f16 != 0, kscale, K, M, xi, rs, ex, part));
     st = run_matmul(ctx, fn, rp, ctx->ones, xi, ctx->ones, rs, nullptr, N, K, M4, yp);
     if (st != NNHIP_OK) return st;
     NNHIP_LAUNCH(fn, launch_digit_combine(ctx->stream, yp, tau, ex, static_cast<const uint32_t*>(rp), B, b_f16 != 0,

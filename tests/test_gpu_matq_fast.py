@@ -373,3 +373,35 @@ def test_matmul_f_split_k_specials(ctx, orc):
     assert np.all(got[::2, 0] == np.inf) and np.all(got[1::2, 0] == -np.inf) and np.all(np.isnan(got[:, 1]))
     assert np.all(got[:, 2] == 0.0)
     assert same_bits(got[:, 3:], digit_model(orc.trits_of(wq, K), X[:, 3:], tau=tau))
+
+
+@pytest.mark.parametrize("b16", [False, True])
+@pytest.mark.parametrize("N,K,M", [(48, 6900, 65), (100, 4097, 64), (37, 2560, 130), (33, 129, 2100), (300, 5000, 7)])
+def test_matmul_f_many_tokens_bits(ctx, orc, N, K, M, b16):
+    """Past a few tokens the digits are made 64 tokens and 128 columns at a time, their absmax in
+    pieces of K: tails of both, f16 inputs, and special tokens among finite ones, bit for bit the
+    digit model; the transposed product (tau folded in per k) on the same shapes."""
+    import torch
+    say(f"ternary_matmul_f many tokens N={N} K={K} M={M} b16={b16}")
+    wq, tau, rp = case(ctx, orc, N, K, seed=N + K + M)
+    X = normal((K, M), 80 + M)
+    X[:, ::3] *= 29.0
+    X[K - 1, 1] = 250.0                        # a token's largest value in its last column
+    X[:, 2] = 0.0
+    X[K // 2, 5] = np.nan
+    X[0, M - 1] = np.inf
+    if b16:
+        X = X.astype(np.float16).astype(np.float32)
+    Xd = dev(X).to(torch.float16) if b16 else dev(X)
+    bad = [5, M - 1]
+    fin = np.setdiff1d(np.arange(M), bad)
+    got = host(ctx.ternary_matmul_f(rp, dev(tau), Xd, N, K))
+    assert same_bits(got[:, fin], digit_model(orc.trits_of(wq, K), X[:, fin], tau=tau))
+    check(got[:, bad], orc.matmul_q(wq, tau, np.ascontiguousarray(X[:, bad]), K), TOL)
+    got16 = ctx.ternary_matmul_f(rp, dev(tau), Xd, N, K, out_f16=True).cpu().numpy()
+    assert same_bits(got16, got.astype(np.float16))
+    A, tauT, At, rpT = transposed_case(ctx, orc, K, N, seed=K + 7 * N + M)
+    got = host(ctx.ternary_matmul_t_f(rpT, dev(tauT), Xd, N))
+    trT = orc.trits_of(At.cpu().numpy().view(np.uint32), K)
+    assert same_bits(got[:, fin], digit_model(trT, X[:, fin], kscale=tauT))
+    check(got[:, bad], orc.matmul_q_t(A, tauT, np.ascontiguousarray(X[:, bad]), N), TOL)
