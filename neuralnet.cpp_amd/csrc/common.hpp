@@ -99,6 +99,16 @@ struct GemvProblem
     const float* res;     // deep decode GEMV: residual (N, M) added after the epilogue (may alias y), or null
 };
 
+// Outputs of a digit product (float activations as four int8 digit tokens each, k_digits.hip): the
+// problem's tokens are the 4M digit rows, its tau may be null (unit), s and y are unused.
+constexpr int32_t kDigitSpecial = 0x7FFFFFFF;  // ex[m] of a token with a NaN or an infinity
+struct DigitOut
+{
+    const int32_t* ex;  // per-token exponent E (|x| < 2^E)
+    void* y;            // (N, M) f32 or f16
+    int32_t y16;
+};
+
 // ---- gated activations (shared by k_glu.hip and the GEMM epilogue)
 // exp(x) from IEEE-rounded operations in a fixed order (no fused multiply-add): Cody-Waite
 // reduction x = k ln2 + r with ln2 split as 22713/32768 + fl(ln2 - 22713/32768) (the first
@@ -267,6 +277,7 @@ hipError_t launch_gemv_grouped(hipStream_t st, const GemvProblem* d_probs, const
 size_t gemv_grid_waves(size_t n_items, int num_cus, bool lds);
 // Prefill GEMM; tile is one of NNHIP_GEMM_TILE_* (AUTO: gemm_tile_choice).
 hipError_t launch_gemm(hipStream_t st, const GemvProblem& p, int num_cus, int tile);
+hipError_t launch_gemm_digits(hipStream_t st, const GemvProblem& p, const DigitOut& g, int num_cus, int tile);
 int gemm_tile_choice(const GemvProblem& p, int num_cus);
 // Time of one round of 128 x 128 / 64 x 64 blocks relative to one round of 256 x 128 blocks,
 // measured over M = 128..4096, K = 2560..6912, N = 2560..13824 (with these the automatic choice
@@ -292,8 +303,16 @@ hipError_t launch_glu_interleave(hipStream_t st, const uint32_t* wq, const float
 // (4 int8 digit tokens per token, row sums, per-token exponents) and the int64 combine
 // kscale (nullable, per k) multiplies the activations first (the transposed product's tau);
 // tau (nullable) is the per-row output factor.
+// Where the digit kernels write the outputs of the special tokens (Y null: left to the combine)
+struct DigitSpecials
+{
+    const uint32_t* rp;
+    const float* tau;  // per output row, or null (unit)
+    void* y;           // (N, M)
+    int32_t N, y16;
+};
 hipError_t launch_digits(hipStream_t st, const void* B, bool b16, const float* kscale, size_t K, size_t M, int8_t* xi,
-                         int32_t* rowsum, int32_t* ex, uint32_t* part);
+                         int32_t* rowsum, int32_t* ex, uint32_t* part, const DigitSpecials& sp);
 size_t digit_part_bytes(size_t M);  // part: pieces of the tokens' absmax
 hipError_t launch_digit_combine(hipStream_t st, const float* Yp, const float* tau, const int32_t* ex,
                                 const uint32_t* rp, const void* B, bool b16, const float* kscale, size_t N, size_t K,

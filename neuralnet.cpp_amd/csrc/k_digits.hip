@@ -7,12 +7,13 @@
 // digits X = d0 + 256 d1 + 65536 d2 + 2^24 d3, every d in [-128, 127]. The digits are four int8
 // "tokens" 4m .. 4m+3 for the ternary x int8 GEMV / GEMM, whose int32 sums are exact; run with
 // unit scales its outputs are the exact integers A_p = sum_k trit * d_p (|A_p| <= 128 K < 2^24
-// while K < 131072). The combine kernel forms T = sum_p A_p 256^p in int64 (exact) and
-// Y = tau * (fl(T) * 2^(E_m - 30)): the only roundings are x to the fixed-point grid
+// while K < 131072). The combine forms T = sum_p A_p 256^p (exact) and
+// Y = tau * (fl(T) * 2^(E_m - 30)), in the GEMM's epilogue for M > 4 tokens (k_gemm.hip; K <= 65280),
+// else in kernels here: the only roundings are x to the fixed-point grid
 // (<= 2^(E_m - 31) per element), the conversion of T and the multiply by tau — far inside the
 // reference tolerance of f32 accumulation (1e-4 x max(1, max|Y|), src/ternary_gemm_test.cpp:503-516).
-// A token holding NaN or +-inf takes an exact IEEE path in the combine kernel instead (per row:
-// NaN if any NaN term, 0 x inf term or opposite infinities, else the infinity's sign), which is
+// A token holding NaN or +-inf takes an exact IEEE path instead (in the combine kernel, or in the
+// digit kernels where the GEMM combines; per row: NaN if any NaN term, 0 x inf term or opposite infinities, else the infinity's sign), which is
 // what the reference's per-term products give.
 #include "common.hpp"
 #include "gemv_tile.hpp"
@@ -25,7 +26,6 @@ namespace
 {
 
 constexpr int kDigBlock = 256;
-constexpr int32_t kSpecialToken = 0x7FFFFFFF;  // ex[m] of a token with a NaN or an infinity
 
 __device__ __forceinline__ float load_b(const void* B, size_t idx, bool f16)
 {
@@ -40,6 +40,50 @@ __device__ __forceinline__ float load_bk(const void* B, const float* kscale, int
     return kscale ? __fmul_rn(kscale[k], x) : x;
 }
 
+// Code (trit + 2) of row n, column k in the T16K256 layout.
+__device__ __forceinline__ int code_at(const uint32_t* rp, int KT, int n, int k)
+{
+    const int rt = n >> 4, r = n & 15, kt = k >> 8, kk = k & 255;
+    const int j = kk >> 6, g = (kk >> 4) & 3, q = (kk >> 2) & 3, b = kk & 3;
+    const uint32_t word = rp[((size_t)rt * KT + kt) * 256 + 4 * (16 * g + r) + q];
+    return (int)((word >> (8 * b + 2 * j)) & 3u);
+}
+
+// Y[n, m] of a token holding a NaN or an infinity: the finite terms cannot change a NaN or an
+// infinite total, so only the non-finite ones are evaluated (IEEE products tau_n * trit * x):
+// NaN if any is NaN (0 x inf included) or infinities of both signs meet, else that infinity.
+__device__ float special_dot(const void* B, bool b16, const float* kscale, const uint32_t* rp, int KT, int K, int M,
+                             int n, int m, float tn)
+{
+    bool nan = false, pos = false, neg = false;
+    for (int k = 0; k < K; ++k)
+    {
+        const float x = load_bk(B, kscale, k, M, m, b16);
+        if (fabsf(x) <= 3.4028234663852886e38f) continue;
+        const float tw = tn * (float)(code_at(rp, KT, n, k) - 2);
+        if (x != x || tw != tw || tw == 0.0f)
+            nan = true;
+        else if ((tw > 0.0f) == (x > 0.0f))
+            pos = true;
+        else
+            neg = true;
+    }
+    return (nan || (pos && neg)) ? __builtin_nanf("") : (pos ? __builtin_inff() : -__builtin_inff());
+}
+
+// A special token's outputs for rows n0, n0 + step, ... (the GEMM epilogue leaves them alone)
+__device__ void write_specials(const DigitSpecials& sp, const void* B, bool b16, const float* kscale, int K, int Kp, int M,
+                               int m, int n0, int step)
+{
+    for (int n = n0; n < sp.N; n += step)
+    {
+        const float y = special_dot(B, b16, kscale, sp.rp, Kp / kTileK, K, M, n, m, sp.tau ? sp.tau[n] : 1.0f);
+        const size_t o = (size_t)n * M + m;
+        if (sp.y16) reinterpret_cast<_Float16*>(sp.y)[o] = (_Float16)y;
+        else reinterpret_cast<float*>(sp.y)[o] = y;
+    }
+}
+
 // One block per token: absmax (and non-finite detection), then the four digit rows. Each thread
 // takes columns k = tid + kDigThreads * (8 i + u), eight independent loads in flight per step.
 constexpr int kDigThreads = 1024;
@@ -48,7 +92,7 @@ constexpr int kDigUnroll = 8;
 __global__ __launch_bounds__(kDigThreads) void k_digits(const void* __restrict__ B, bool f16,
                                                         const float* __restrict__ kscale, int K, int M, int Kp,
                                                         int8_t* __restrict__ xi, int32_t* __restrict__ rowsum,
-                                                        int32_t* __restrict__ ex)
+                                                        int32_t* __restrict__ ex, DigitSpecials sp)
 {
     constexpr int NW = kDigThreads / kWave;
     __shared__ float smax[NW];
@@ -140,7 +184,8 @@ __global__ __launch_bounds__(kDigThreads) void k_digits(const void* __restrict__
         for (int i = 0; i < NW; ++i) t += ssum[tid][i];
         rowsum[4 * m + tid] = t;
     }
-    if (tid == 0) ex[m] = bad ? kSpecialToken : E;
+    if (tid == 0) ex[m] = bad ? kDigitSpecial : E;
+    if (bad && sp.y) write_specials(sp, B, f16, kscale, K, Kp, M, m, tid, kDigThreads);
 }
 
 // The digits of many tokens (M > 4) in two launches that read B along tokens, 64 at a time, so
@@ -210,7 +255,7 @@ __global__ __launch_bounds__(kDigRowThreads) void k_digit_rows(const void* __res
                                                                const float* __restrict__ kscale, int K, int M, int Kp,
                                                                const uint32_t* __restrict__ part, int parts,
                                                                int8_t* __restrict__ xi, int32_t* __restrict__ rowsum,
-                                                               int32_t* __restrict__ ex)
+                                                               int32_t* __restrict__ ex, DigitSpecials sp)
 {
     constexpr int NW = kDigRowThreads / kWave, KW = kDigCols / NW;  // columns per wave
     // token t's four digit rows of the block's columns, 32 words each; one word more per token, so
@@ -233,7 +278,7 @@ __global__ __launch_bounds__(kDigRowThreads) void k_digit_rows(const void* __res
     const bool bad = mx >= 0x7F800000u;  // an infinity or a NaN: all digits 0
     int E = 0;
     if (!bad) (void)frexpf(__builtin_bit_cast(float, mx), &E);  // |x| < 2^E (E = 0 for a zero token)
-    if (blockIdx.y == 0 && w == 0 && m < M) ex[m] = bad ? kSpecialToken : E;
+    if (blockIdx.y == 0 && w == 0 && m < M) ex[m] = bad ? kDigitSpecial : E;
     const int shift = 30 - E;
     int s[4] = {0, 0, 0, 0};
 #pragma unroll
@@ -276,6 +321,9 @@ __global__ __launch_bounds__(kDigRowThreads) void k_digit_rows(const void* __res
     const int p = w;  // one digit per wave
     if (m < M)
         atomicAdd(&rowsum[4 * m + p], ssum[0][p][lane] + ssum[1][p][lane] + ssum[2][p][lane] + ssum[3][p][lane]);
+    // the rows of a special token, shared out over the blocks of its tokens
+    if (sp.y && m < M && bad)
+        write_specials(sp, B, sizeof(BT) == 2, kscale, K, Kp, M, m, blockIdx.y * NW + w, gridDim.y * NW);
 }
 
 // The same digits for a few long tokens (the split-k path, M <= 4): block (c, m) takes columns
@@ -371,38 +419,7 @@ __global__ __launch_bounds__(kChunkThreads) void k_digits_chunks(const void* __r
         for (int i = 0; i < NW; ++i) t += ssum[tid][i];
         rsp[((size_t)m * P + c) * 4 + tid] = t;
     }
-    if (c == 0 && tid == 0) ex[m] = bad ? kSpecialToken : E;
-}
-
-// Code (trit + 2) of row n, column k in the T16K256 layout.
-__device__ __forceinline__ int code_at(const uint32_t* rp, int KT, int n, int k)
-{
-    const int rt = n >> 4, r = n & 15, kt = k >> 8, kk = k & 255;
-    const int j = kk >> 6, g = (kk >> 4) & 3, q = (kk >> 2) & 3, b = kk & 3;
-    const uint32_t word = rp[((size_t)rt * KT + kt) * 256 + 4 * (16 * g + r) + q];
-    return (int)((word >> (8 * b + 2 * j)) & 3u);
-}
-
-// Y[n, m] of a token holding a NaN or an infinity: the finite terms cannot change a NaN or an
-// infinite total, so only the non-finite ones are evaluated (IEEE products tau_n * trit * x):
-// NaN if any is NaN (0 x inf included) or infinities of both signs meet, else that infinity.
-__device__ float special_dot(const void* B, bool b16, const float* kscale, const uint32_t* rp, int KT, int K, int M,
-                             int n, int m, float tn)
-{
-    bool nan = false, pos = false, neg = false;
-    for (int k = 0; k < K; ++k)
-    {
-        const float x = load_bk(B, kscale, k, M, m, b16);
-        if (fabsf(x) <= 3.4028234663852886e38f) continue;
-        const float tw = tn * (float)(code_at(rp, KT, n, k) - 2);
-        if (x != x || tw != tw || tw == 0.0f)
-            nan = true;
-        else if ((tw > 0.0f) == (x > 0.0f))
-            pos = true;
-        else
-            neg = true;
-    }
-    return (nan || (pos && neg)) ? __builtin_nanf("") : (pos ? __builtin_inff() : -__builtin_inff());
+    if (c == 0 && tid == 0) ex[m] = bad ? kDigitSpecial : E;
 }
 
 // Y[n, m] from the digit products Yp (N, 4M): tau[n] * (fl(T) * 2^(E_m - 30)); a special token
@@ -420,7 +437,7 @@ __global__ __launch_bounds__(kDigBlock) void k_digit_combine(const float* __rest
     const int E = ex[m];
     const float tn = tau ? tau[n] : 1.0f;
     float y;
-    if (E != kSpecialToken)
+    if (E != kDigitSpecial)
     {
         const float4 d = *reinterpret_cast<const float4*>(Yp + ((size_t)n * M + m) * 4);
         const long long T = (long long)d.x + ((long long)d.y << 8) + ((long long)d.z << 16) + ((long long)d.w << 24);
@@ -453,7 +470,7 @@ __global__ __launch_bounds__(kDigBlock) void k_digit_combine_parts(const int32_t
     const int E = ex[m];
     const float tn = tau ? tau[n] : 1.0f;
     float y;
-    if (E != kSpecialToken)
+    if (E != kDigitSpecial)
     {
         long long T = 0;
 #pragma unroll
@@ -758,7 +775,7 @@ namespace
 
 template <typename BT, bool KS>
 hipError_t launch_digits_tok(hipStream_t st, const void* B, const float* kscale, size_t K, size_t M, int8_t* xi,
-                             int32_t* rowsum, int32_t* ex, uint32_t* part)
+                             int32_t* rowsum, int32_t* ex, uint32_t* part, const DigitSpecials& sp)
 {
     const size_t Kp = round_up(K, kTileK);
     const unsigned tiles = (unsigned)ceil_div(M, (size_t)kDigTok);
@@ -768,7 +785,7 @@ hipError_t launch_digits_tok(hipStream_t st, const void* B, const float* kscale,
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL((k_digit_rows<BT, KS>), dim3(tiles, (unsigned)(Kp / kDigCols)), dim3(kDigRowThreads), 0, st, B,
-                       kscale, (int)K, (int)M, (int)Kp, part, (int)parts, xi, rowsum, ex);
+                       kscale, (int)K, (int)M, (int)Kp, part, (int)parts, xi, rowsum, ex, sp);
     return hipGetLastError();
 }
 
@@ -777,23 +794,23 @@ hipError_t launch_digits_tok(hipStream_t st, const void* B, const float* kscale,
 size_t digit_part_bytes(size_t M) { return (size_t)kDigParts * M * 4; }
 
 hipError_t launch_digits(hipStream_t st, const void* B, bool b16, const float* kscale, size_t K, size_t M, int8_t* xi,
-                         int32_t* rowsum, int32_t* ex, uint32_t* part)
+                         int32_t* rowsum, int32_t* ex, uint32_t* part, const DigitSpecials& sp)
 {
     const size_t Kp = round_up(K, kTileK);
-    // one launch, one block per token, while the column reads stay few: a lone call of the two
-    // launches takes 1-2 us longer there (K=2560, whole product: M=40 23.4 against 24.6 us, M=256
-    // 44.5 against 42.1; K=1000, M=256 15.5 against 16.6; K=6912: M=5 26.0 against 28.1, M=8 29.4
-    // against 28.3)
+    // one launch, one block per token, while the column reads stay few: there a lone call of the two
+    // launches takes 1-2 us longer (whole product before the fused combine, one against two launches:
+    // K=2560 M=40 23.4 / 24.6 us, M=256 44.5 / 42.1; K=1000 M=256 15.5 / 16.6; K=6912 M=5 26.0 /
+    // 28.1, M=8 29.4 / 28.3)
     if (M <= 6 || (K <= 4096 && K * M <= (size_t(1) << 18)))
     {
-        k_digits<<<dim3((unsigned)M), kDigThreads, 0, st>>>(B, b16, kscale, (int)K, (int)M, (int)Kp, xi, rowsum, ex);
+        k_digits<<<dim3((unsigned)M), kDigThreads, 0, st>>>(B, b16, kscale, (int)K, (int)M, (int)Kp, xi, rowsum, ex, sp);
         return hipGetLastError();
     }
     if (b16)
-        return kscale ? launch_digits_tok<_Float16, true>(st, B, kscale, K, M, xi, rowsum, ex, part)
-                      : launch_digits_tok<_Float16, false>(st, B, kscale, K, M, xi, rowsum, ex, part);
-    return kscale ? launch_digits_tok<float, true>(st, B, kscale, K, M, xi, rowsum, ex, part)
-                  : launch_digits_tok<float, false>(st, B, kscale, K, M, xi, rowsum, ex, part);
+        return kscale ? launch_digits_tok<_Float16, true>(st, B, kscale, K, M, xi, rowsum, ex, part, sp)
+                      : launch_digits_tok<_Float16, false>(st, B, kscale, K, M, xi, rowsum, ex, part, sp);
+    return kscale ? launch_digits_tok<float, true>(st, B, kscale, K, M, xi, rowsum, ex, part, sp)
+                  : launch_digits_tok<float, false>(st, B, kscale, K, M, xi, rowsum, ex, part, sp);
 }
 
 size_t digit_chunks(size_t K) { return ceil_div(round_up(K, kTileK), (size_t)kChunk); }

@@ -41,6 +41,17 @@
 // of a SIMD stay level instead of the older one finishing first and idling at the barrier.
 // The epilogue operands (tau, s, rowsum, bias) are loaded before the k-split exchange.
 //
+// Digit products (launch_gemm_digits, k_gemm_digits): the tokens are the int8 digit rows 4m + p of
+// float activations (k_digits.hip), and the epilogue adds the four digit sums of a token
+// (T = sum_p A_p 256^p) and stores tau * (fl(T) * 2^(E - 30)) instead of 4 x N x M exact integers
+// as f32, which a second kernel read back (226 MB each way for 6912 x 2048). A quad of lanes holds
+// the four digits of one token, so the sum is two butterfly steps on the quad. The digit rows go
+// to the MFMA columns in the order that leaves a lane kTB consecutive tokens of one row: one wide
+// store per lane and row, whole lines per instruction. The main loop is the same.
+// The whole product of 2048 f32 tokens (back to back in a graph): 2560 -> 6912 230.1 -> 147.2 us,
+// 6912 -> 2560 185.6 -> 150.9 us, 40 tokens 23.3 -> 18.9 us. Outputs are stored at element
+// alignment, four tokens at once for any M (M=2047: 167.1 us with single stores, 158.4 us so).
+//
 // Block order is XCD-aware: blocks are dealt round-robin to the 8 XCDs, and each XCD gets
 // whole token blocks (all N for them), so a token block's activations stay in that XCD's L2.
 #include "common.hpp"
@@ -250,11 +261,26 @@ struct Gemm
             for (int m = 0; m < kMs; ++m) dst[rb][m] = *reinterpret_cast<const v4i*>(p + rb * 2048 + m * 512);
     }
 
-    // B fragments of one step for the wave's kTB token blocks (32 token rows = 8 KiB apart)
+    // B fragments of one step for the wave's kTB token blocks: column c of block n is token row
+    // 32 n + c; with kDig (digit products) row 4 kTB (c / 4) + 4 n + c % 4
+    template <bool kDig>
     static __device__ __forceinline__ void read_b(v4i (&dst)[kTB], const uint8_t* p)
     {
 #pragma unroll
-        for (int n = 0; n < kTB; ++n) dst[n] = *reinterpret_cast<const v4i*>(p + n * 32 * kTileK);
+        for (int n = 0; n < kTB; ++n) dst[n] = *reinterpret_cast<const v4i*>(p + n * (kDig ? 4 : 32) * kTileK);
+    }
+
+    // The token row (within the wave's) of column c of block 0, and the swizzle key of a token row:
+    // its column mod 16, so that the 16 columns of a read fall on 16 distinct chunk positions.
+    template <bool kDig>
+    static __device__ __forceinline__ int col_row(int c)
+    {
+        return kDig ? 4 * kTB * (c >> 2) + (c & 3) : c;
+    }
+    template <bool kDig>
+    static __device__ __forceinline__ int row_key(int row)
+    {
+        return kDig ? ((row / (4 * kTB)) & 3) * 4 + (row & 3) : row & 15;
     }
 
     struct Lane
@@ -266,7 +292,7 @@ struct Gemm
 
     // One stage: the wave's 32-k steps (all eight, or the four of its k half). P selects the
     // register set holding this stage's A words; the next stage's go to the other set.
-    template <int P>
+    template <bool kDig, int P>
     static __device__ __forceinline__ void run_stage(int s, int KT, uint8_t* lds, const Dma& d, const Lane& ln,
                                               v4i (&wa)[2][kRB][kMs], v4i (&bf)[2][kTB], v16i (&acc)[kRB][kTB])
     {
@@ -278,7 +304,7 @@ struct Gemm
             const int cur = i & 1, nxt = cur ^ 1;
             if (i + 1 < kWaveSteps)
             {
-                read_b(bf[nxt], slot + ln.b_off + ln.b_step[i + 1]);
+                read_b<kDig>(bf[nxt], slot + ln.b_off + ln.b_step[i + 1]);
             }
             else if (s + 1 < KT)
             {
@@ -288,7 +314,7 @@ struct Gemm
                 if (s + kSlots < KT) issue_loads(lds, d, s % kSlots, s + kSlots, KT, 0, kPartLoads);
                 const uint8_t* nslot = lds + ((s + 1) % kSlots) * kSlotBytes;
                 read_a(wa[P ^ 1], nslot + ln.a_off);
-                read_b(bf[nxt], nslot + ln.b_off + ln.b_step[0]);
+                read_b<kDig>(bf[nxt], nslot + ln.b_off + ln.b_step[0]);
             }
             __builtin_amdgcn_sched_barrier(0);
             step_prio(i == kWaveSteps - 1 ? 0 : i + 1);
@@ -557,8 +583,126 @@ struct Gemm
         }
     }
 
-    static __device__ __forceinline__ void body(const GemvProblem& p, int n_mblocks, int n_nblocks, int xcd_mode,
-                                                bool h_keep)
+    // Epilogue operands of a digit product, per lane: column 4q + c of block n is digit c of token
+    // t0 + n, t0 = tok_w / 4 + kTB q, and after the quad sums the lane holds row 8j + 4h + c of each
+    // 32-row block for j = 0..3.
+    struct DigOps
+    {
+        int nrs[kTB];      // -2 rowsum of the lane's digit rows, shifted as the sums are
+        int ex[kTB];       // the tokens' exponents
+        float tv[kRBf][4]; // tau of the lane's output rows
+    };
+
+    static __device__ __forceinline__ void load_dig(const GemvProblem& p, const DigitOut& g, DigOps& e, int rb0, int row_w,
+                                                    int t0, int h, int c)
+    {
+        const __amdgpu_buffer_rsrc_t rrs = rsrc(p.rowsum, (uint32_t)p.M * 4u);
+        const __amdgpu_buffer_rsrc_t rex = rsrc(g.ex, (uint32_t)p.M);  // M / 4 tokens
+        const __amdgpu_buffer_rsrc_t rtau = rsrc(p.tau ? (const void*)p.tau : (const void*)g.ex, p.tau ? (uint32_t)p.N * 4u : 0u);
+#pragma unroll
+        for (int n = 0; n < kTB; ++n)
+        {
+            const uint32_t m = (uint32_t)(4 * (t0 + n) + c);
+            e.nrs[n] = -(2 * __builtin_bit_cast(int, __builtin_amdgcn_raw_buffer_load_b32(rrs, m * 4u, 0, 0))) * (1 << (8 * (c & 1)));
+            e.ex[n] = __builtin_bit_cast(int, __builtin_amdgcn_raw_buffer_load_b32(rex, (uint32_t)(t0 + n) * 4u, 0, 0));
+        }
+#pragma unroll
+        for (int r = 0; r < kRBf; ++r)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+            {
+                const uint32_t row = (uint32_t)(row_w + (rb0 + r) * 32 + 8 * j + 4 * h + c);
+                const float t = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rtau, row * 4u, 0, 0));
+                e.tv[r][j] = p.tau ? t : 1.0f;
+            }
+    }
+
+    // T = sum_p A_p 256^p per (row, token) over the lane quad, then y = tau * (fl(T) * 2^(E - 30)).
+    // Lane c holds A_c of rows 0..3 (of each group of four) and ends with row c: the xor-1 step adds
+    // A_0 + 256 A_1 or A_2 + 256 A_3 (below 2^31 while K <= 65280), the xor-2 step brings the other
+    // half. H 2^16 + L is exact in f64, so its conversion is the one rounding of fl(T). Special
+    // tokens (k_digits.hip has written their rows) and tokens past M are not stored.
+    static __device__ __forceinline__ void store_dig(const GemvProblem& p, const DigitOut& g, const v16i (&acc)[kRB][kTB],
+                                                     const DigOps& e, int rb0, int nrb, int row_w, int t0, int h, int c)
+    {
+        const int M = p.M >> 2, sh = 8 * (c & 1);
+        const bool odd = c & 1, high = c & 2;
+        const double s_keep = high ? 65536.0 : 1.0, s_recv = high ? 1.0 : 65536.0;
+        bool ok[kTB], all = true;
+#pragma unroll
+        for (int n = 0; n < kTB; ++n)
+        {
+            ok[n] = t0 + n < M && e.ex[n] != kDigitSpecial;
+            all = all && ok[n];
+        }
+#pragma unroll
+        for (int rb = 0; rb < kRB; ++rb)
+        {
+            if (rb < rb0 || rb >= rb0 + nrb) continue;
+            const int r = epi_slot(rb);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+            {
+                const int row = row_w + rb * 32 + 8 * j + 4 * h + c;
+                float y[kTB];
+#pragma unroll
+                for (int n = 0; n < kTB; ++n)
+                {
+                    int a[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) a[i] = (acc[rb][n][4 * j + i] << sh) + e.nrs[n];
+                    // quad_perm [1,0,3,2] and [2,3,0,1]
+                    const int u = (odd ? a[1] : a[0]) + __builtin_amdgcn_mov_dpp(odd ? a[0] : a[1], 0xB1, 0xF, 0xF, true);
+                    const int v = (odd ? a[3] : a[2]) + __builtin_amdgcn_mov_dpp(odd ? a[2] : a[3], 0xB1, 0xF, 0xF, true);
+                    const int keep = high ? v : u, recv = __builtin_amdgcn_mov_dpp(high ? u : v, 0x4E, 0xF, 0xF, true);
+                    const double T = __builtin_fma((double)keep, s_keep, (double)recv * s_recv);
+                    y[n] = e.tv[r][j] * __builtin_ldexpf((float)T, e.ex[n] - 30);
+                }
+                if (row >= p.N) continue;
+                const size_t at = (size_t)row * (size_t)M + (size_t)t0;
+                if (g.y16)
+                {
+                    typedef _Float16 vh __attribute__((ext_vector_type(kTB), aligned(2)));  // M may be odd
+                    _Float16* dst = static_cast<_Float16*>(g.y) + at;
+                    if (all)
+                    {
+                        vh w;
+#pragma unroll
+                        for (int n = 0; n < kTB; ++n) w[n] = (_Float16)y[n];
+                        *reinterpret_cast<vh*>(dst) = w;
+                    }
+                    else
+                    {
+#pragma unroll
+                        for (int n = 0; n < kTB; ++n)
+                            if (ok[n]) dst[n] = (_Float16)y[n];
+                    }
+                }
+                else
+                {
+                    typedef float vf __attribute__((ext_vector_type(kTB), aligned(4)));  // M may be odd
+                    float* dst = static_cast<float*>(g.y) + at;
+                    if (all)
+                    {
+                        vf w;
+#pragma unroll
+                        for (int n = 0; n < kTB; ++n) w[n] = y[n];
+                        *reinterpret_cast<vf*>(dst) = w;
+                    }
+                    else
+                    {
+#pragma unroll
+                        for (int n = 0; n < kTB; ++n)
+                            if (ok[n]) dst[n] = y[n];
+                    }
+                }
+            }
+        }
+    }
+
+    template <bool kDig>
+    static __device__ __forceinline__ void body(const GemvProblem& p, const DigitOut& g, int n_mblocks, int n_nblocks,
+                                                int xcd_mode, bool h_keep)
     {
         extern __shared__ __align__(16) uint8_t lds[];
         const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -596,7 +740,7 @@ struct Gemm
         {
             const int row = (wave * kBDma + i) * 4 + (lane >> 4);  // token row within the block
             const int pos = lane & 15;                             // chunk position in the LDS row
-            const int c = pos ^ (row & 15);                        // global chunk stored there
+            const int c = pos ^ row_key<kDig>(row);                // global chunk stored there
             const int m = m0 + row;
             d.b_voff[i] = m < p.M ? (uint32_t)m * Kp + (uint32_t)c * 16u : 0x80000000u;
         }
@@ -606,8 +750,8 @@ struct Gemm
         Lane ln;
         ln.a_off = (uint32_t)((wn * (kWaveRows / 16) + (l32 >> 4)) * 1024 + (16 * h + (l32 & 15)) * 16 +
                               (kKSplit == 2 ? ks * 512 : 0));
-        ln.b_off = (uint32_t)(kABytes + (wm * kWaveToks + l32) * kTileK);
-        const int rsw = h ^ (l32 & 15);  // token row % 16 is l32 % 16 for every token block
+        ln.b_off = (uint32_t)(kABytes + (wm * kWaveToks + col_row<kDig>(l32)) * kTileK);
+        const int rsw = h ^ (l32 & 15);  // the key of the lane's token row in every token block
 #pragma unroll
         for (int i = 0; i < kWaveSteps; ++i)
         {
@@ -632,15 +776,15 @@ struct Gemm
         v4i wa[2][kRB][kMs];
         v4i bf[2][kTB];
         read_a(wa[0], lds + ln.a_off);
-        read_b(bf[0], lds + ln.b_off + ln.b_step[0]);
+        read_b<kDig>(bf[0], lds + ln.b_off + ln.b_step[0]);
 
         int s = 0;
         for (; s + 1 < KT; s += 2)
         {
-            run_stage<0>(s, KT, lds, d, ln, wa, bf, acc);
-            run_stage<1>(s + 1, KT, lds, d, ln, wa, bf, acc);
+            run_stage<kDig, 0>(s, KT, lds, d, ln, wa, bf, acc);
+            run_stage<kDig, 1>(s + 1, KT, lds, d, ln, wa, bf, acc);
         }
-        if (s < KT) run_stage<0>(s, KT, lds, d, ln, wa, bf, acc);
+        if (s < KT) run_stage<kDig, 0>(s, KT, lds, d, ln, wa, bf, acc);
 
         // ---- epilogue operands (issued before the k-split exchange, whose LDS round trip hides
         // their latency), then the exchange: the two waves of a pair swap partial sums through LDS;
@@ -656,7 +800,10 @@ struct Gemm
         wait_lgkm0();
         wait_vmcnt<0>();
         EpiOps e;
-        load_epilogue(p, e, rb0, row_w, tok_w, h, l32);
+        DigOps de;
+        const int dig_t0 = tok_w / 4 + kTB * (l32 >> 2);
+        if constexpr (kDig) load_dig(p, g, de, rb0, row_w, dig_t0, h, l32 & 3);
+        else load_epilogue(p, e, rb0, row_w, tok_w, h, l32);
         if (kKSplit == 2)
         {
             lds_barrier();  // every wave is done with the ring
@@ -668,6 +815,11 @@ struct Gemm
         }
 
         // ---- epilogue
+        if constexpr (kDig)
+        {
+            store_dig(p, g, acc, de, rb0, nrb, row_w, dig_t0, h, l32 & 3);
+            return;
+        }
         const bool full = rt0 * 16 + kBN <= p.N && m0 + kBM <= p.M;
         if (p.glu)
         {
@@ -691,7 +843,14 @@ template <class G>
 __global__ __launch_bounds__(G::kThreads) __attribute__((amdgpu_waves_per_eu(G::kWavesPerSimd, G::kWavesPerSimd))) void
 k_gemm(GemvProblem p, int n_mblocks, int n_nblocks, int xcd_mode, int h_keep)
 {
-    G::body(p, n_mblocks, n_nblocks, xcd_mode, h_keep != 0);
+    G::template body<false>(p, DigitOut{}, n_mblocks, n_nblocks, xcd_mode, h_keep != 0);
+}
+
+template <class G>
+__global__ __launch_bounds__(G::kThreads) __attribute__((amdgpu_waves_per_eu(G::kWavesPerSimd, G::kWavesPerSimd))) void
+k_gemm_digits(GemvProblem p, DigitOut g, int n_mblocks, int n_nblocks, int xcd_mode)
+{
+    G::template body<true>(p, g, n_mblocks, n_nblocks, xcd_mode, false);
 }
 
 }  // namespace
@@ -707,22 +866,28 @@ using GemmA = Gemm<256, 128, NNHIP_GEMM_WAVES_N, NNHIP_GEMM_WAVES_M, NNHIP_GEMM_
 using GemmB = Gemm<128, 128, 2, 2, 2, 3>;
 using GemmC = Gemm<64, 64, 2, 2, 1, 6>;
 
+// dig: the digit product's outputs, or null for the int8 product
 template <class G>
-hipError_t launch_cfg(hipStream_t st, const GemvProblem& p, bool h_keep)
+hipError_t launch_cfg(hipStream_t st, const GemvProblem& p, bool h_keep, const DigitOut* dig)
 {
-    static bool attr_set = false;
-    if (!attr_set)
+    static bool attr_set[2] = {false, false};
+    bool& set = attr_set[dig ? 1 : 0];
+    if (!set)
     {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm<G>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, G::kLdsBytes);
+        const void* fn = dig ? reinterpret_cast<const void*>(&k_gemm_digits<G>) : reinterpret_cast<const void*>(&k_gemm<G>);
+        const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, G::kLdsBytes);
         if (e != hipSuccess) return e;
-        attr_set = true;
+        set = true;
     }
     const int n_mblocks = (int)ceil_div((size_t)p.M, G::kBM);
     const int n_nblocks = (int)ceil_div((size_t)p.N, G::kBN);
     const int xcd_mode = (n_mblocks % 8 == 0) ? 1 : 0;
     const unsigned blocks = (unsigned)(n_mblocks * n_nblocks);
-    hipLaunchKernelGGL(k_gemm<G>, dim3(blocks), dim3(G::kThreads), G::kLdsBytes, st, p, n_mblocks, n_nblocks,
+    if (dig)
+        hipLaunchKernelGGL(k_gemm_digits<G>, dim3(blocks), dim3(G::kThreads), G::kLdsBytes, st, p, *dig, n_mblocks,
+                           n_nblocks, xcd_mode);
+    else
+        hipLaunchKernelGGL(k_gemm<G>, dim3(blocks), dim3(G::kThreads), G::kLdsBytes, st, p, n_mblocks, n_nblocks,
                        xcd_mode, h_keep ? 1 : 0);
     return hipGetLastError();
 }
@@ -758,7 +923,7 @@ GemvProblem gemm_rows_from(const GemvProblem& p, int rows0)
     GemvProblem q = p;
     const size_t rt0 = (size_t)rows0 / 16;
     q.rp = p.rp + rt0 * (size_t)p.KT * 64;  // 1024 bytes = 64 x 16 per (row tile, k tile)
-    q.tau = p.tau + rows0;
+    if (p.tau) q.tau = p.tau + rows0;
     if (p.bias) q.bias = p.bias + rows0;
     q.N = p.N - rows0;
     if (p.glu)
@@ -766,7 +931,7 @@ GemvProblem gemm_rows_from(const GemvProblem& p, int rows0)
         q.glu_F = p.glu_F - rows0 / 2;
         q.y = p.y + (size_t)(rows0 / 2) * (size_t)p.M;
     }
-    else
+    else if (p.y)  // (a digit product's outputs are not p.y)
     {
         q.y = p.y + (size_t)rows0 * (size_t)p.M;
         if (p.res) q.res = p.res + (size_t)rows0 * (size_t)p.M;
@@ -801,16 +966,14 @@ GemmSplit gemm_split_choice(const GemvProblem& p, int num_cus)
 namespace
 {
 
-hipError_t launch_tile(hipStream_t st, const GemvProblem& p, int tile, bool h_keep)
+hipError_t launch_tile(hipStream_t st, const GemvProblem& p, int tile, bool h_keep, const DigitOut* dig)
 {
-    if (tile == NNHIP_GEMM_TILE_128x128) return launch_cfg<GemmB>(st, p, h_keep);
-    if (tile == NNHIP_GEMM_TILE_64x64) return launch_cfg<GemmC>(st, p, h_keep);
-    return launch_cfg<GemmA>(st, p, h_keep);
+    if (tile == NNHIP_GEMM_TILE_128x128) return launch_cfg<GemmB>(st, p, h_keep, dig);
+    if (tile == NNHIP_GEMM_TILE_64x64) return launch_cfg<GemmC>(st, p, h_keep, dig);
+    return launch_cfg<GemmA>(st, p, h_keep, dig);
 }
 
-}  // namespace
-
-hipError_t launch_gemm(hipStream_t st, const GemvProblem& p, int num_cus, int tile)
+hipError_t launch_any(hipStream_t st, const GemvProblem& p, int num_cus, int tile, const DigitOut* dig)
 {
     if (p.N == 0 || p.M == 0) return hipSuccess;
     const bool h_keep = p.glu && (size_t)p.glu_F * (size_t)p.M * 4 <= kGemmHKeepBytes;
@@ -819,16 +982,34 @@ hipError_t launch_gemm(hipStream_t st, const GemvProblem& p, int num_cus, int ti
         const GemmSplit s = gemm_split_choice(p, num_cus);
         if (s.rows > 0)
         {
-            GemvProblem head = p;
+            GemvProblem head = p, tail = gemm_rows_from(p, s.rows);
             head.N = s.rows;
             if (p.glu) head.glu_F = s.rows / 2;
-            const hipError_t e = launch_cfg<GemmA>(st, head, h_keep);
+            const hipError_t e = launch_cfg<GemmA>(st, head, h_keep, dig);
             if (e != hipSuccess) return e;
-            return launch_tile(st, gemm_rows_from(p, s.rows), s.tail_tile, h_keep);
+            DigitOut rest{};
+            if (dig)
+            {
+                rest = *dig;
+                rest.y = static_cast<uint8_t*>(dig->y) + (size_t)s.rows * (size_t)(p.M / 4) * (dig->y16 ? 2 : 4);
+            }
+            return launch_tile(st, tail, s.tail_tile, h_keep, dig ? &rest : nullptr);
         }
         tile = s.tile;
     }
-    return launch_tile(st, p, tile, h_keep);
+    return launch_tile(st, p, tile, h_keep, dig);
+}
+
+}  // namespace
+
+hipError_t launch_gemm(hipStream_t st, const GemvProblem& p, int num_cus, int tile)
+{
+    return launch_any(st, p, num_cus, tile, nullptr);
+}
+
+hipError_t launch_gemm_digits(hipStream_t st, const GemvProblem& p, const DigitOut& g, int num_cus, int tile)
+{
+    return launch_any(st, p, num_cus, tile, &g);
 }
 
 }  // namespace nnhip
