@@ -15,22 +15,34 @@
 // token column m = b*T + t (the BitLinear outputs of the B*T tokens); caches (B, max_len,
 // Hkv*dk) as the decode step's; cos / sin (max_len, dk/2).
 //
-// k_attn_prefill: work-group = (32 queries, KV head g, sequence b) with one wave per query head
-// of the group (R = H / Hkv waves), so each 32-key tile of K and V is staged in LDS once for all
-// R heads. Per 32-key tile a wave computes S^T = K . Q^T (32 keys x 32 queries) on the fp32 MFMA
-// v_mfma_f32_32x32x2_f32, folds it into an online softmax (running max and sum per query), and
-// accumulates O^T += V^T . P^T. With S^T (not S) in the accumulators, lane l holds query l % 32
-// and keys 8(v/4) + 4(l/32) + v%4 of its 16 elements v, which is exactly the B operand of the
-// P . V products (lane l, k = l/32) when the keys of product s are taken in that order; the
-// A operand of product s is then V[key][dimension] of that key for the lane's dimension. The sum
-// over the head dimension in S^T takes product s = 4c + e over dimensions 8c + e and 8c + 4 + e
-// (the two lane halves), which a lane reads as one 16-byte chunk of its K row. K and V rows are
-// padded to dk + 4 floats in LDS, so the 16-byte reads of 8 consecutive rows cover all banks.
+// k_attn_prefill: the fp32 MFMA's rate (157 TFLOP/s) bounded this attention (101 of it at 4 x 2048
+// tokens), and the f16 MFMA runs 16 times as fast. So the products run on v_mfma_f32_32x32x16_f16
+// with every f32 operand as the sum of two f16 halves, x 2^e = hi + lo: e brings the operand's
+// largest value (of a query; of a tile of K; of V so far) to 2^14..2^15, hi and lo are rounded to
+// nearest, so the pair holds x to 2^-24 of itself (to 2^-39 of the largest value for elements far
+// below it). Products of halves are exact in f32; low x low (below 2^-24 of a term) is left out:
+// three MFMAs per product with f32 caches, two with f16 caches, whose elements are halves as they
+// are. Sums, softmax and output are f32, and sums of 16 products at a time round less often than
+// the fp32 MFMA's pairs: against float64, 4 x 2048 tokens of 20 heads over 5 KV heads of 128 are
+// 4.6e-7 off (f32 products: 6.7e-7), 3 x 1111 at position 517 6.7e-7 (9.7e-7).
+// What the halves cannot hold (infinities, NaN, a tile's largest value outside 2^+-48) sends the
+// work-group to the f32 products (attend_f32).
+//
+// Work-group = 8 waves = (the R = H / Hkv heads of KV head g) x (8 / R blocks of 32 queries) of
+// sequence b; all waves share each 32-key tile of K and V, staged in LDS as f16 planes (double
+// buffered, one barrier per tile): the next tile is converted from registers while the one after
+// it is loaded. A wave computes S^T = K . Q^T (32 keys x 32 queries) and O^T += V^T . P^T, where
+// lane l holds query l % 32 throughout: its 16 elements v of S^T are keys 8(v/4) + 4(l/32) + v%4,
+// and V^T is staged with its keys in that order, so P^T is an operand as it stands. Row 32d + r of
+// V^T is dimension (DK/32) r + d, which lets a staging lane load contiguous dimensions and its
+// stores fall on all banks. K rows and V^T rows are XOR-swizzled in 16-byte chunks.
+// Softmax in log2 units with the hardware exp2; a query's reference maximum moves only when it has
+// grown by 2^8 (probabilities are held times 2^6, at most 2^14), so the sums are rarely rescaled.
 // Work-groups are issued heaviest first (the last query blocks attend over the most keys).
-// f32 throughout; the accumulation order differs from a sequential dot product (results within
-// 2e-6 relative of a float64 evaluation on the test data). Caches of f16 elements (compute = F16)
-// are widened exactly when a tile is staged; the fill rounds the rotated keys and the values to
-// the nearest f16 (ties to even), as the decode append does.
+// Measured (calls back to back, us, f32 products / here): f32 caches 4 x 2048 tokens 848 / 372,
+// 3 x 1111 at 517 432 / 186, 16 x 2048 3077 / 1242; f16 caches 821 / 235, 426 / 125, 3132 / 866.
+// Caches of f16 elements (compute = F16): the fill rounds the rotated keys and the values to the
+// nearest f16 (ties to even), as the decode append does.
 #include "common.hpp"
 
 #include <cmath>
@@ -129,6 +141,17 @@ __global__ __launch_bounds__(256) void k_kv_fill(const float* __restrict__ k, co
 
 // ------------------------------------------------------------------ causal attention
 
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+
+constexpr int kPWaves = 8;             // waves of a work-group: R heads x (8 / R) blocks of 32 queries
+constexpr int kPThreads = 64 * kPWaves;
+constexpr int kPExpMax = 48;           // scalings beyond 2^+-48 take the f32 products
+constexpr float kPLazy = 8.0f;         // log2 growth of a query's maximum before its sums are rescaled
+constexpr float kPBias = 6.0f;         // probabilities are held times 2^6: at most 2^14 with the growth
+
 struct PrefillArgs
 {
     const float* q;
@@ -139,120 +162,139 @@ struct PrefillArgs
     float* out;
     int B, T, H, Hkv, R, pos0, max_len, nqb;
     float scale;
-};
-
-template <int DK>
-struct PrefillTile
-{
-    static constexpr int KROW = DK + 4;  // padded K / V row (floats)
-    static constexpr int kFloats = 2 * kPK * KROW;
-    static constexpr int kBytes = 2 * kFloats * 4;  // double-buffered
+    float scale2;  // |scale| * log2(e)
+    int f32;       // 1: the f32 products throughout (a scale outside [2^-20, 2^20])
 };
 
 template <int DK, typename CT>
-__global__ __launch_bounds__(512) void k_attn_prefill(PrefillArgs a)
+struct PrefillTile
+{
+    static constexpr int kPlanes = sizeof(CT) == 4 ? 2 : 1;  // high and low f16 halves of f32 values
+    static constexpr int kPlane = kPK * DK * 2;              // bytes of one plane of K or of V
+    static constexpr int kBuf = 2 * kPlanes * kPlane;        // K planes, then V planes
+    static constexpr int KROW = DK + 4;                      // f32 products: padded row (floats)
+    static constexpr int kF32 = 2 * kPK * KROW * 4;
+    static constexpr int kMain = 2 * kBuf > kF32 ? 2 * kBuf : kF32;  // double-buffered
+    static constexpr int kBytes = kMain + 128;               // maxima of two tiles, the fallback flag
+};
+
+// The two halves of four f32 values scaled into f16's range: x = hi + lo up to 2^-24 |x| or 2^-25
+__device__ __forceinline__ void split2(float x0, float x1, v2h& hi, v2h& lo)
+{
+    hi = __builtin_convertvector(v2f{x0, x1}, v2h);
+    // one fma each: the differences are exact
+    lo = __builtin_convertvector(v2f{__builtin_fmaf((float)hi[0], -1.0f, x0), __builtin_fmaf((float)hi[1], -1.0f, x1)}, v2h);
+}
+
+// 2^e for |e| <= 126
+__device__ __forceinline__ float pow2(int e) { return __builtin_bit_cast(float, (uint32_t)(127 + e) << 23); }
+
+// The exponent that brings values whose largest bit pattern is mx (sign cleared) into [2^14, 2^15):
+// 0 for all-zero values. Outside +-kPExpMax (infinities and NaN among it) the f32 products run.
+__device__ __forceinline__ int f16_exp(uint32_t mx) { return mx == 0 ? 0 : 14 + 127 - (int)(mx >> 23); }
+
+// The wave's largest value
+__device__ __forceinline__ uint32_t wave_max(uint32_t v)
+{
+    for (int off = 32; off >= 1; off >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, off, kWave));
+    return v;
+}
+
+// Where a wave works: query head, first query, the lane's query
+struct PrefillWave
+{
+    int b, g, head, t0, qt, qpos;
+    bool live;  // the wave has queries
+};
+
+// The lane's rotated query value pairs, f(dimension, value, value of dimension + DK/2) for its
+// dimensions below DK/2: those with (i / G) % 2 == h in groups of G
+template <int DK, int G, typename F>
+__device__ __forceinline__ void load_query(const PrefillArgs& a, const PrefillWave& w, int h, F&& f)
 {
     constexpr int HALF = DK / 2;
-    constexpr int NC = DK / 8;    // 16-byte chunks of a lane half's K row (S products in groups of 4)
-    constexpr int ND = DK / 32;   // 32-row blocks of O^T
-    constexpr int KROW = PrefillTile<DK>::KROW;
-    constexpr int TILE = PrefillTile<DK>::kFloats;
-    extern __shared__ __align__(16) float smem[];
-
-    const int nthreads = a.R * 64;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, h = lane >> 5, l32 = lane & 31;
-    // heaviest items first: query block from the last one down
-    const int per_qb = a.B * a.Hkv;
-    const int qb = a.nqb - 1 - (int)blockIdx.x / per_qb;
-    const int bg = (int)blockIdx.x % per_qb;
-    const int b = bg / a.Hkv, g = bg % a.Hkv;
-    const int head = g * a.R + wave;
     const int M = a.B * a.T;
-    const int t0 = qb * kPQ;
-    const int qt = t0 + l32;                  // this lane's query token (valid if < T)
-    const int qpos = a.pos0 + qt;             // its position
-    const int row = a.Hkv * DK;
-    const int valid = a.pos0 + a.T;           // cache rows [0, valid) hold keys / values
-
-    // ---- the lane's rotated query values: qv[4c + e] = rot(q)[8c + 4h + e]
-    float qv[DK / 2];
+    const __amdgpu_buffer_rsrc_t rq = pf_rsrc(a.q, (uint32_t)((size_t)a.H * DK * (size_t)M * 4u));
+    const __amdgpu_buffer_rsrc_t rc = pf_rsrc(a.cosT ? a.cosT : a.q, a.cosT ? (uint32_t)((size_t)a.max_len * HALF * 4u) : 0u);
+    const __amdgpu_buffer_rsrc_t rs = pf_rsrc(a.cosT ? a.sinT : a.q, a.cosT ? (uint32_t)((size_t)a.max_len * HALF * 4u) : 0u);
+    const bool qok = w.qt < a.T;
+    const int m = w.b * a.T + w.qt;
+#pragma unroll
+    for (int c = 0; c < HALF / (2 * G); ++c)
     {
-        const __amdgpu_buffer_rsrc_t rq = pf_rsrc(a.q, (uint32_t)((size_t)a.H * DK * (size_t)M * 4u));
-        const int m = b * a.T + qt;
-        const bool qok = qt < a.T;
-        float x[DK / 2];
+        float x0[G], x1[G], cs[G], sn[G];
 #pragma unroll
-        for (int c = 0; c < NC; ++c)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-            {
-                const int i = 8 * c + 4 * h + e;
-                const uint32_t off = qok ? (uint32_t)(((size_t)(head * DK + i) * (size_t)M + (size_t)m) * 4u) : 0x80000000u;
-                x[4 * c + e] = ld_f(rq, off);
-            }
-        if (a.cosT)
+        for (int e = 0; e < G; ++e)
         {
-            const __amdgpu_buffer_rsrc_t rc = pf_rsrc(a.cosT, (uint32_t)((size_t)a.max_len * HALF * 4u));
-            const __amdgpu_buffer_rsrc_t rs = pf_rsrc(a.sinT, (uint32_t)((size_t)a.max_len * HALF * 4u));
-            // dimension i < HALF pairs with i + HALF: chunk c pairs with c + NC/2 in the same lane
-#pragma unroll
-            for (int c = 0; c < NC / 2; ++c)
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                {
-                    const int j = 8 * c + 4 * h + e;
-                    const uint32_t off = qok ? (uint32_t)(((size_t)qpos * HALF + (size_t)j) * 4u) : 0x80000000u;
-                    const float cs = ld_f(rc, off), sn = ld_f(rs, off);
-                    pf_rope(x[4 * c + e], x[4 * (c + NC / 2) + e], cs, sn, qv[4 * c + e], qv[4 * (c + NC / 2) + e]);
-                }
+            const int i = 2 * G * c + G * h + e;
+            const size_t at = ((size_t)(w.head * DK + i) * (size_t)M + (size_t)m) * 4u;
+            x0[e] = ld_f(rq, qok ? (uint32_t)at : 0x80000000u);
+            x1[e] = ld_f(rq, qok ? (uint32_t)(at + (size_t)HALF * (size_t)M * 4u) : 0x80000000u);
+            const uint32_t off = qok ? (uint32_t)(((size_t)w.qpos * HALF + (size_t)i) * 4u) : 0x80000000u;
+            cs[e] = ld_f(rc, off);
+            sn[e] = ld_f(rs, off);
         }
-        else
-        {
 #pragma unroll
-            for (int i = 0; i < DK / 2; ++i) qv[i] = x[i];
+        for (int e = 0; e < G; ++e)
+        {
+            float y0 = x0[e], y1 = x1[e];
+            if (a.cosT) pf_rope(x0[e], x1[e], cs[e], sn[e], y0, y1);
+            f(c, e, y0, y1);
         }
     }
+}
 
-    // ---- key tiles: keys [0, last] with last = min(qpos of the block's last query, valid - 1)
-    const int last_key = min(a.pos0 + min(t0 + kPQ, a.T) - 1, valid - 1);
-    const int nkb = last_key / kPK + 1;
-    const size_t seq_off = (size_t)b * (size_t)a.max_len * (size_t)row;
-    // rows at or past `valid` (and past max_len) read as zeros: their scores are masked and their
-    // zero values keep 0 * v finite
-    const uint32_t seq_bytes = (uint32_t)((size_t)min(valid, a.max_len) * (size_t)row * sizeof(CT));
-    const __amdgpu_buffer_rsrc_t rk = pf_rsrc(static_cast<const CT*>(a.kc) + seq_off, seq_bytes);
-    const __amdgpu_buffer_rsrc_t rv = pf_rsrc(static_cast<const CT*>(a.vc) + seq_off, seq_bytes);
+// out[head*DK + i][m] for the lane's query: element v of block d belongs to row r = 8(v/4) + 4h + v%4
+// of the block; dim(d, r) is its dimension
+template <int DK, typename D>
+__device__ __forceinline__ void store_out(const PrefillArgs& a, const PrefillWave& w, const v16f* o, float l, int e, int h,
+                                          D&& dim)
+{
+    if (w.qt >= a.T) return;
+    const int M = a.B * a.T, m = w.b * a.T + w.qt;
+#pragma unroll
+    for (int d = 0; d < DK / 32; ++d)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+            a.out[(size_t)(w.head * DK + dim(d, 8 * (v >> 2) + 4 * h + (v & 3))) * (size_t)M + (size_t)m] =
+                ldexpf(o[d][v] / l, -e);
+}
 
-    // staging: float4 units of a 32 x DK tile, spread over the work-group's threads
-    constexpr int kUnits = kPK * DK / 4;
-    auto stage_tile = [&](int kb, float* tile) {
-        float* ks = tile;
-        float* vs = tile + kPK * KROW;
-        for (int u = tid; u < kUnits; u += nthreads)
-        {
-            const int key = u / (DK / 4), c4 = u % (DK / 4);
-            const uint32_t off =
-                (uint32_t)(((size_t)(kb * kPK + key) * (size_t)row + (size_t)g * DK + 4 * c4) * sizeof(CT));
-            const float4 kk = ld_c4<CT>(rk, off);
-            const float4 vv = ld_c4<CT>(rv, off);
-            *reinterpret_cast<float4*>(ks + key * KROW + 4 * c4) = kk;
-            *reinterpret_cast<float4*>(vs + key * KROW + 4 * c4) = vv;
-        }
-    };
-
+// The work-group's attention on the fp32 MFMA (v_mfma_f32_32x32x2_f32), for inputs that the f16
+// halves cannot hold: infinities, NaN, or a tile whose largest value is outside 2^+-48. Per 32-key
+// tile S^T (not S) is in the accumulators, so lane l holds query l % 32 and keys
+// 8(v/4) + 4(l/32) + v%4 of its 16 elements v: the B operand of the P . V products when the keys of
+// product s are taken in that order. The sum over the head dimension takes product s = 4c + e over
+// dimensions 8c + e and 8c + 4 + e (the two lane halves).
+template <int DK, typename CT>
+__device__ void attend_f32(const PrefillArgs& a, const PrefillWave& w, int last_key, __amdgpu_buffer_rsrc_t rk,
+                           __amdgpu_buffer_rsrc_t rv, float* ks)
+{
+    constexpr int NC = DK / 8, ND = DK / 32, KROW = PrefillTile<DK, CT>::KROW;
+    const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, l32 = lane & 31;
+    const int row = a.Hkv * DK;
+    float* vs = ks + kPK * KROW;
+    float qv[DK / 2];  // qv[4c + e] = rotated query value of dimension 8c + 4h + e
+    load_query<DK, 4>(a, w, h, [&](int c, int e, float y0, float y1) {
+        qv[4 * c + e] = y0;
+        qv[4 * (c + NC / 2) + e] = y1;
+    });
     v16f o[ND];
 #pragma unroll
     for (int d = 0; d < ND; ++d) o[d] = v16f{};
     float m_run = -__builtin_inff(), l_run = 0.0f;
-
-    stage_tile(0, smem);
-    __syncthreads();
-    for (int kb = 0; kb < nkb; ++kb)
+    for (int kb = 0; kb <= last_key / kPK; ++kb)
     {
-        const float* tile = smem + (kb & 1) * TILE;
-        const float* ks = tile;
-        const float* vs = tile + kPK * KROW;
-        // S^T = K . Q^T over the head dimension
+        __syncthreads();  // every wave is done with the previous tile
+        for (int u = tid; u < kPK * DK / 4; u += kPThreads)
+        {
+            const int key = u / (DK / 4), c4 = u % (DK / 4);
+            const uint32_t off = (uint32_t)(((size_t)(kb * kPK + key) * (size_t)row + (size_t)w.g * DK + 4 * c4) * sizeof(CT));
+            *reinterpret_cast<float4*>(ks + key * KROW + 4 * c4) = ld_c4<CT>(rk, off);
+            *reinterpret_cast<float4*>(vs + key * KROW + 4 * c4) = ld_c4<CT>(rv, off);
+        }
+        __syncthreads();
+        if (!w.live || kb * kPK > a.pos0 + w.t0 + kPQ - 1) continue;
         v16f s = v16f{};
 #pragma unroll
         for (int c = 0; c < NC; ++c)
@@ -263,31 +305,15 @@ __global__ __launch_bounds__(512) void k_attn_prefill(PrefillArgs a)
             s = __builtin_amdgcn_mfma_f32_32x32x2f32(kk.z, qv[4 * c + 2], s, 0, 0, 0);
             s = __builtin_amdgcn_mfma_f32_32x32x2f32(kk.w, qv[4 * c + 3], s, 0, 0, 0);
         }
-        // the next tile's loads overlap this tile's softmax and products
-        if (kb + 1 < nkb) stage_tile(kb + 1, smem + ((kb + 1) & 1) * TILE);
-        // online softmax over this tile's keys (element v: key 32kb + 8(v/4) + 4h + v%4); the
-        // causal mask only where the tile reaches past the wave's first query
         float sc[16];
         float mx = -__builtin_inff();
-        if (kb * kPK + kPK - 1 <= a.pos0 + t0)
-        {
 #pragma unroll
-            for (int v = 0; v < 16; ++v)
-            {
-                sc[v] = s[v] * a.scale;
-                mx = fmaxf(mx, sc[v]);
-            }
-        }
-        else
+        for (int v = 0; v < 16; ++v)
         {
-#pragma unroll
-            for (int v = 0; v < 16; ++v)
-            {
-                const int key = kb * kPK + 8 * (v >> 2) + 4 * h + (v & 3);
-                const float x = s[v] * a.scale;
-                sc[v] = key <= qpos ? x : -__builtin_inff();
-                mx = fmaxf(mx, sc[v]);
-            }
+            const int key = kb * kPK + 8 * (v >> 2) + 4 * h + (v & 3);
+            const float x = s[v] * a.scale;
+            sc[v] = key <= w.qpos ? x : -__builtin_inff();
+            mx = fmaxf(mx, sc[v]);
         }
         mx = fmaxf(mx, __shfl_xor(mx, 32));
         const float m_new = fmaxf(m_run, mx);
@@ -303,8 +329,7 @@ __global__ __launch_bounds__(512) void k_attn_prefill(PrefillArgs a)
         ls += __shfl_xor(ls, 32);
         l_run = l_run * corr + ls;
         m_run = m_new;
-        // corr is exactly 1 where the running maximum did not move: skip the rescale when that
-        // holds for every lane (multiplying by 1 would change no bit)
+        // corr is exactly 1 where the running maximum did not move
         if (__builtin_amdgcn_ballot_w64(corr != 1.0f) != 0)
         {
 #pragma unroll
@@ -312,7 +337,6 @@ __global__ __launch_bounds__(512) void k_attn_prefill(PrefillArgs a)
 #pragma unroll
                 for (int v = 0; v < 16; ++v) o[d][v] *= corr;
         }
-        // O^T += V^T . P^T: product s takes key 8(s/4) + 4h + s%4 (the lane's score element s)
 #pragma unroll
         for (int d = 0; d < ND; ++d)
 #pragma unroll
@@ -321,37 +345,413 @@ __global__ __launch_bounds__(512) void k_attn_prefill(PrefillArgs a)
                 const int key = 8 * (sp >> 2) + 4 * h + (sp & 3);
                 o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(vs[key * KROW + 32 * d + l32], sc[sp], o[d], 0, 0, 0);
             }
-        __syncthreads();  // every wave is done with this tile; the next one is in LDS
     }
+    if (w.live) store_out<DK>(a, w, o, l_run, 0, h, [](int d, int r) { return 32 * d + r; });
+}
 
-    // ---- out[head*dk + i][m] = O^T[i][query] / l for the block's valid queries
-    if (qt < a.T)
-    {
-        const int m = b * a.T + qt;
+template <int DK, typename CT>
+__global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
+{
+    using Tile = PrefillTile<DK, CT>;
+    constexpr bool F32C = sizeof(CT) == 4;
+    constexpr int NC = DK / 16;  // MFMA steps over the head dimension
+    constexpr int ND = DK / 32;  // 32-row blocks of O^T, and dimensions per lane when staging V
+    constexpr int CH = DK / 8;   // 16-byte chunks of a K row
+    constexpr int KU = CH * kPK / 256;  // chunks a thread stages
+    extern __shared__ __align__(16) uint8_t smem[];
+    uint32_t* smax = reinterpret_cast<uint32_t*>(smem + Tile::kMain);  // [2][8]: per tile parity and wave
+    // set to send the work-group to the f32 products: written in iteration kb (or before the loop) into
+    // [(kb + 1) & 1] and read after the barrier of iteration kb + 1, so all waves read the same value
+    int* sflag = reinterpret_cast<int*>(smem + Tile::kMain + 64);
+
+    const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, l32 = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // heaviest items first: the last queries attend over the most keys
+    const int per_qb = a.B * a.Hkv;
+    const int qb = a.nqb - 1 - (int)blockIdx.x / per_qb;
+    const int bg = (int)blockIdx.x % per_qb;
+    PrefillWave w;
+    w.b = bg / a.Hkv;
+    w.g = bg % a.Hkv;
+    w.head = w.g * a.R + wave % a.R;
+    const int qn = kPQ * (kPWaves / a.R);  // queries of the work-group
+    w.t0 = qb * qn + wave / a.R * kPQ;
+    w.qt = w.t0 + l32;
+    w.qpos = a.pos0 + w.qt;
+    w.live = w.t0 < a.T;
+    const int row = a.Hkv * DK;
+    const int valid = a.pos0 + a.T;  // cache rows [0, valid) hold keys / values
+    const int last_key = a.pos0 + min(qb * qn + qn, a.T) - 1;
+    const int nkb = last_key / kPK + 1;
+    const size_t seq_off = (size_t)w.b * (size_t)a.max_len * (size_t)row;
+    // rows at or past `valid` read as zeros: their scores are masked and their zero values keep
+    // 0 * v finite
+    const uint32_t seq_bytes = (uint32_t)((size_t)min(valid, a.max_len) * (size_t)row * sizeof(CT));
+    const __amdgpu_buffer_rsrc_t rk = pf_rsrc(static_cast<const CT*>(a.kc) + seq_off, seq_bytes);
+    const __amdgpu_buffer_rsrc_t rv = pf_rsrc(static_cast<const CT*>(a.vc) + seq_off, seq_bytes);
+
+    if (tid < 2) sflag[tid] = tid == 0 ? a.f32 : 0;
+    __syncthreads();
+
+    // ---- staging, 16 elements per thread: waves 0-3 take V (thread = 4 keys x ND dimensions), waves
+    // 4-7 take K (thread = KU chunks of 8 dimensions of a key). raw holds them as loaded.
+    constexpr int RW = F32C ? 16 : 8;  // words
+    uint32_t raw[RW];
+    const bool is_v = wave < 4;
+    const int u = tid & 255;
+    const int vq = u >> 5, vg = u & 31;  // V: key quad, dimension group
+    auto load_raw = [&](int kb) {
+        if (is_v)
+        {
 #pragma unroll
-        for (int d = 0; d < ND; ++d)
-#pragma unroll
-            for (int v = 0; v < 16; ++v)
+            for (int i = 0; i < 4; ++i)
             {
-                const int i = 32 * d + 8 * (v >> 2) + 4 * h + (v & 3);
-                a.out[(size_t)(head * DK + i) * (size_t)M + (size_t)m] = o[d][v] / l_run;
+                const uint32_t off = (uint32_t)(((size_t)(kb * kPK + 4 * vq + i) * (size_t)row + (size_t)w.g * DK + ND * vg) * sizeof(CT));
+                constexpr int W = ND * (int)sizeof(CT) / 4;  // words per key
+                if constexpr (W == 4)
+                {
+                    const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(rv, off, 0, 0);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) raw[4 * i + e] = x[e];
+                }
+                else if constexpr (W == 2)
+                {
+                    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+                    const u32x2 x = __builtin_amdgcn_raw_buffer_load_b64(rv, off, 0, 0);
+                    raw[2 * i] = x[0];
+                    raw[2 * i + 1] = x[1];
+                }
+                else raw[i] = __builtin_amdgcn_raw_buffer_load_b32(rv, off, 0, 0);
+            }
+        }
+        else
+        {
+#pragma unroll
+            for (int j = 0; j < KU; ++j)
+            {
+                const int ct = u + 256 * j;
+                const uint32_t off = (uint32_t)(((size_t)(kb * kPK + ct / CH) * (size_t)row + (size_t)w.g * DK + 8 * (ct % CH)) * sizeof(CT));
+#pragma unroll
+                for (int q = 0; q < (F32C ? 2 : 1); ++q)
+                {
+                    const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(rk, off + 16 * q, 0, 0);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) raw[(F32C ? 8 : 4) * j + 4 * q + e] = x[e];
+                }
+            }
+        }
+    };
+    // words of raw in use
+    constexpr int VW = 4 * ND * (int)sizeof(CT) / 4, KW = KU * 8 * (int)sizeof(CT) / 4;
+    static_assert(VW == KW && VW <= RW, "V and K threads stage the same amount");
+    // f32: the wave's largest magnitude for the tile's scaling; f16: only whether all are finite
+    auto post_max = [&](int kb, int* flag) {
+        uint32_t mx = 0;
+        if constexpr (F32C)
+        {
+#pragma unroll
+            for (int e = 0; e < VW; ++e) mx = max(mx, raw[e] & 0x7FFFFFFFu);
+            mx = wave_max(mx);
+            if (lane == 0) smax[(kb & 1) * 8 + wave] = mx;
+        }
+        else
+        {
+#pragma unroll
+            for (int e = 0; e < VW; ++e)
+            {
+                mx = max(mx, raw[e] & 0x7FFFu);
+                mx = max(mx, (raw[e] >> 16) & 0x7FFFu);
+            }
+            if (__builtin_amdgcn_ballot_w64(mx >= 0x7C00u) != 0 && lane == 0) *flag = 1;
+        }
+    };
+    int ek = 0, ev = 1 << 20;  // exponents of the staged tile: K's own, V's running smallest
+    // the tile's exponents, then raw as f16 halves into buffer kb & 1
+    auto convert = [&](int kb, int* flag) {
+        uint8_t* buf = smem + (kb & 1) * Tile::kBuf;
+        if constexpr (F32C)
+        {
+            const uint32_t* sm = smax + (kb & 1) * 8;
+            const uint32_t mv = max(max(sm[0], sm[1]), max(sm[2], sm[3])), mk = max(max(sm[4], sm[5]), max(sm[6], sm[7]));
+            ek = __builtin_amdgcn_readfirstlane(f16_exp(mk));
+            const int e = __builtin_amdgcn_readfirstlane(f16_exp(mv));
+            if (mv != 0) ev = min(ev, e);
+            if (abs(ek) > kPExpMax || abs(e) > kPExpMax)
+            {
+                if (tid == 0) *flag = 1;
+                ek = ev = 0;
+            }
+        }
+        const float sv = F32C ? pow2(ev > kPExpMax ? 0 : ev) : 1.0f, sk = F32C ? pow2(ek) : 1.0f;
+        if (is_v)
+        {
+            // row 32e + vg = dimension ND vg + e; its 4 chunks are (16-key half s, lane half) and hold
+            // keys 16s + 8a + 4h + i in the order (a, i): the accumulators' order of S^T
+            const int s = vq >> 2, ah = (vq >> 1) & 1, hh = vq & 1;
+#pragma unroll
+            for (int e = 0; e < ND; ++e)
+            {
+                const int r = 32 * e + vg;
+                uint8_t* dst = buf + Tile::kPlanes * Tile::kPlane + r * 64 + (((2 * s + hh) ^ ((r >> 2) & 3)) << 4) + 8 * ah;
+                if constexpr (F32C)
+                {
+                    float x[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) x[i] = __builtin_bit_cast(float, raw[ND * i + e]) * sv;
+                    v2h h0, h1, l0, l1;
+                    split2(x[0], x[1], h0, l0);
+                    split2(x[2], x[3], h1, l1);
+                    *reinterpret_cast<v4h*>(dst) = v4h{h0[0], h0[1], h1[0], h1[1]};
+                    *reinterpret_cast<v4h*>(dst + Tile::kPlane) = v4h{l0[0], l0[1], l1[0], l1[1]};
+                }
+                else
+                {
+                    // half e of each key's words
+                    constexpr int W = ND / 2;
+                    const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
+                    uint32_t* d = reinterpret_cast<uint32_t*>(dst);
+                    d[0] = __builtin_amdgcn_perm(raw[W + e / 2], raw[e / 2], sel);
+                    d[1] = __builtin_amdgcn_perm(raw[3 * W + e / 2], raw[2 * W + e / 2], sel);
+                }
+            }
+        }
+        else
+        {
+#pragma unroll
+            for (int j = 0; j < KU; ++j)
+            {
+                const int ct = u + 256 * j, key = ct / CH, c = ct % CH;
+                uint8_t* dst = buf + key * DK * 2 + ((c ^ (CH == 16 ? key & 15 : (key >> 1) & 7)) << 4);
+                if constexpr (F32C)
+                {
+                    v8h hi, lo;
+#pragma unroll
+                    for (int e = 0; e < 8; e += 2)
+                    {
+                        v2h x, y;
+                        split2(__builtin_bit_cast(float, raw[8 * j + e]) * sk, __builtin_bit_cast(float, raw[8 * j + e + 1]) * sk, x, y);
+                        hi[e] = x[0], hi[e + 1] = x[1];
+                        lo[e] = y[0], lo[e + 1] = y[1];
+                    }
+                    *reinterpret_cast<v8h*>(dst) = hi;
+                    *reinterpret_cast<v8h*>(dst + Tile::kPlane) = lo;
+                }
+                else
+                    *reinterpret_cast<u32x4*>(dst) = u32x4{raw[4 * j], raw[4 * j + 1], raw[4 * j + 2], raw[4 * j + 3]};
+            }
+        }
+    };
+
+    // Fragments from LDS, four 16-byte reads at a time, a group ahead of the products that use them:
+    // group g of K holds steps GS g .., group g of V^T (block, half) pairs GS g .., each with its low
+    // plane next to it for f32 caches. The chunk swizzles are XORs of address bits that no other term
+    // of the offset reaches.
+    constexpr int GS = 4 / Tile::kPlanes;
+    static_assert(NC % GS == 0 && (2 * ND) % GS == 0, "whole groups");
+    const uint32_t k_at = (uint32_t)(l32 * DK * 2 + ((h ^ (CH == 16 ? l32 & 15 : (l32 >> 1) & 7)) << 4));
+    const uint32_t v_at = (uint32_t)(Tile::kPlanes * Tile::kPlane + l32 * 64 + ((h ^ ((l32 >> 2) & 3)) << 4));
+    auto read_k = [&](v8h(&f)[4], uint32_t par, int g) {
+#pragma unroll
+        for (int e = 0; e < GS; ++e)
+        {
+            const uint8_t* p = smem + ((par + k_at) ^ (uint32_t)((GS * g + e) << 5));
+#pragma unroll
+            for (int q = 0; q < Tile::kPlanes; ++q)
+                f[Tile::kPlanes * e + q] = *reinterpret_cast<const v8h*>(p + q * Tile::kPlane);
+        }
+    };
+    auto read_v = [&](v8h(&f)[4], uint32_t par, int g) {
+#pragma unroll
+        for (int e = 0; e < GS; ++e)
+        {
+            const int d = (GS * g + e) >> 1, t = (GS * g + e) & 1;
+            const uint8_t* p = smem + ((par + v_at) ^ (uint32_t)(t << 5)) + d * 2048;
+#pragma unroll
+            for (int q = 0; q < Tile::kPlanes; ++q)
+                f[Tile::kPlanes * e + q] = *reinterpret_cast<const v8h*>(p + q * Tile::kPlane);
+        }
+    };
+
+    load_raw(0);
+
+    // ---- the lane's rotated query in halves: step c holds dimensions 16c + 8h + 0..7, scaled by 2^eq
+    v8h qh[NC], ql[NC];
+    float eqf = 0.0f;  // 2^-eq |scale| log2(e)
+    if (w.live)
+    {
+        float qv[DK / 2];
+        uint32_t mx = 0;
+        const float sign = a.scale < 0.0f ? -1.0f : 1.0f;
+        load_query<DK, 8>(a, w, h, [&](int c, int e, float y0, float y1) {
+            qv[8 * c + e] = y0;
+            qv[8 * (c + NC / 2) + e] = y1;
+            mx = max(mx, max(__builtin_bit_cast(uint32_t, y0) & 0x7FFFFFFFu, __builtin_bit_cast(uint32_t, y1) & 0x7FFFFFFFu));
+        });
+        mx = max(mx, (uint32_t)__shfl_xor((int)mx, 32, kWave));
+        int eq = f16_exp(mx);
+        const bool far = abs(eq) > kPExpMax;
+        if (__builtin_amdgcn_ballot_w64(far) != 0 && lane == 0) sflag[0] = 1;
+        if (far) eq = 0;
+        const float sq = sign * pow2(eq);
+        eqf = a.scale2 * pow2(-eq);
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int e = 0; e < 8; e += 2)
+            {
+                v2h x, y;
+                split2(qv[8 * c + e] * sq, qv[8 * c + e + 1] * sq, x, y);
+                qh[c][e] = x[0], qh[c][e + 1] = x[1];
+                ql[c][e] = y[0], ql[c][e + 1] = y[1];
             }
     }
+    v16f o[ND];
+#pragma unroll
+    for (int d = 0; d < ND; ++d) o[d] = v16f{};
+    float m_ref = -__builtin_inff(), l_run = 0.0f;  // log2 units; l_run: this lane half's keys
+    int eo = 0;                                     // the exponent of V in o
+
+    post_max(0, sflag);
+    __syncthreads();
+    convert(0, sflag);
+    if (nkb > 1)
+    {
+        load_raw(1);
+        post_max(1, sflag);
+    }
+    bool fallback = false;
+    for (int kb = 0; kb < nkb; ++kb)
+    {
+        __syncthreads();  // tile kb is in LDS, the maxima of tile kb + 1 too; buffer (kb + 1) & 1 is free
+        if (sflag[kb & 1])
+        {
+            fallback = true;
+            break;
+        }
+        const int ek_now = ek, ev_now = ev;
+        // this tile's first K fragments, in flight during the conversion of the next tile
+        const uint32_t par = (uint32_t)(kb & 1) * Tile::kBuf;
+        v8h fr[2][4];
+        read_k(fr[0], par, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (kb + 1 < nkb)
+        {
+            convert(kb + 1, sflag + ((kb + 1) & 1));
+            if (kb + 2 < nkb) load_raw(kb + 2);  // in flight during this tile's products
+        }
+        if (w.live && kb * kPK <= a.pos0 + w.t0 + kPQ - 1)
+        {
+            // S^T = K . Q^T: the products of the halves but low x low (2^-24 of a term)
+            v16f s = v16f{};
+#pragma unroll
+            for (int g = 0; g < NC / GS; ++g)
+            {
+                if (g + 1 < NC / GS) read_k(fr[(g + 1) & 1], par, g + 1);
+                else read_v(fr[(g + 1) & 1], par, 0);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int e = 0; e < GS; ++e)
+                {
+                    const int c = GS * g + e;
+                    const v8h kh = fr[g & 1][Tile::kPlanes * e];
+                    if constexpr (F32C) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[g & 1][2 * e + 1], qh[c], s, 0, 0, 0);
+                    s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, ql[c], s, 0, 0, 0);
+                    s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, qh[c], s, 0, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            // scores in log2 units are s * f; the causal mask only where the tile reaches past the
+            // wave's first query
+            const float f = F32C ? eqf * pow2(-ek_now) : eqf;
+            if (kb * kPK + kPK - 1 > a.pos0 + w.t0)
+            {
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                    if (kb * kPK + 8 * (v >> 2) + 4 * h + (v & 3) > w.qpos) s[v] = -__builtin_inff();
+            }
+            float mx = s[0];
+#pragma unroll
+            for (int v = 1; v < 16; ++v) mx = fmaxf(mx, s[v]);
+            mx = fmaxf(mx, __shfl_xor(mx, 32)) * f;
+            // the reference of a query moves only when its maximum has grown by 2^8 (or is new)
+            const bool grown = mx > m_ref + kPLazy;
+            if (__builtin_amdgcn_ballot_w64(grown) != 0 || (F32C && ev_now != eo))
+            {
+                const float m_new = grown ? mx : m_ref;
+                float corr = __builtin_amdgcn_exp2f(m_ref - m_new);  // 0 on the first tile
+                l_run *= corr;
+                if (F32C && ev_now != eo)
+                {
+                    // V's exponent went down (the first tile: nothing summed yet)
+                    if (kb > 0) corr *= pow2(max(ev_now - eo, -126));
+                    eo = ev_now;
+                }
+#pragma unroll
+                for (int d = 0; d < ND; ++d)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) o[d][v] *= corr;
+                m_ref = m_new;
+            }
+            const float mb = kPBias - m_ref;
+            v8h ph[2], pl[2];
+#pragma unroll
+            for (int v = 0; v < 16; v += 2)
+            {
+                const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[v], f, mb));
+                const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[v + 1], f, mb));
+                l_run += p0;
+                l_run += p1;
+                v2h x, y;
+                split2(p0, p1, x, y);
+                ph[v >> 3][v & 7] = x[0], ph[v >> 3][(v & 7) + 1] = x[1];
+                pl[v >> 3][v & 7] = y[0], pl[v >> 3][(v & 7) + 1] = y[1];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            // O^T += V^T . P^T
+#pragma unroll
+            for (int g = 0; g < 2 * ND / GS; ++g)
+            {
+                const v8h(&f4)[4] = fr[(NC / GS + g) & 1];
+                if (g + 1 < 2 * ND / GS) read_v(fr[(NC / GS + g + 1) & 1], par, g + 1);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int e = 0; e < GS; ++e)
+                {
+                    const int d = (GS * g + e) >> 1, t = (GS * g + e) & 1;
+                    const v8h vh = f4[Tile::kPlanes * e];
+                    if constexpr (F32C) o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f4[2 * e + 1], ph[t], o[d], 0, 0, 0);
+                    o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, pl[t], o[d], 0, 0, 0);
+                    o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, ph[t], o[d], 0, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if (kb + 2 < nkb) post_max(kb + 2, sflag + ((kb + 1) & 1));
+    }
+    if (fallback)
+    {
+        attend_f32<DK, CT>(a, w, last_key, rk, rv, reinterpret_cast<float*>(smem));
+        return;
+    }
+    l_run += __shfl_xor(l_run, 32);
+    if (w.live)
+        store_out<DK>(a, w, o, l_run, F32C ? eo : 0, h, [](int d, int r) { return ND * r + d; });
 }
 
 template <int DK, typename CT>
 hipError_t launch_prefill_dk(hipStream_t st, const PrefillArgs& a)
 {
+    constexpr int lds = PrefillTile<DK, CT>::kBytes;
     static bool attr_set = false;
     if (!attr_set)
     {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_attn_prefill<DK, CT>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, PrefillTile<DK>::kBytes);
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         if (e != hipSuccess) return e;
         attr_set = true;
     }
     const unsigned blocks = (unsigned)(a.nqb * a.B * a.Hkv);
-    hipLaunchKernelGGL((k_attn_prefill<DK, CT>), dim3(blocks), dim3(a.R * 64), PrefillTile<DK>::kBytes, st, a);
+    hipLaunchKernelGGL((k_attn_prefill<DK, CT>), dim3(blocks), dim3(kPThreads), lds, st, a);
     return hipGetLastError();
 }
 
@@ -392,8 +792,11 @@ hipError_t launch_attn_prefill(hipStream_t st, const float* q, const void* kc, c
                                const float* sinT, size_t max_len, float scale, float* out)
 {
     if (B * T == 0) return hipSuccess;
-    PrefillArgs a{q, kc, vc, cosT, sinT, out, (int)B, (int)T, (int)H, (int)Hkv, (int)(H / Hkv), (int)pos0,
-                  (int)max_len, (int)ceil_div(T, kPQ), scale};
+    const size_t R = H / Hkv;
+    const float mag = std::fabs(scale);
+    const bool f32 = !(mag >= 0x1p-20f && mag <= 0x1p20f);
+    PrefillArgs a{q, kc, vc, cosT, sinT, out, (int)B, (int)T, (int)H, (int)Hkv, (int)R, (int)pos0,
+                  (int)max_len, (int)ceil_div(T, kPQ * (kPWaves / R)), scale, (float)(mag * 1.4426950408889634), f32 ? 1 : 0};
     if (cache_f16)
     {
         if (dk == 64) return launch_prefill_dk<64, _Float16>(st, a);

@@ -353,3 +353,87 @@ def test_prefill_gemm_c5_token_count(ctx, orc, nnhip, N, K, gated):
     assert same_bits(Y[:, m0:m0 + 256], band), "band of 256 tokens differs"
     rows = np.unique(np.concatenate([np.arange(0, N, 97), [N - 1]]))
     assert same_bits(Y[rows], ref(rows, 0, M)), "sampled rows differ"
+
+
+def attend64(q, kc, vc, B, T, H, Hkv, dk, pos0, scale):
+    """Causal attention in float64: q (H*dk, B*T), caches (B, max_len, Hkv*dk) -> (H*dk, B*T), and the
+    largest sum of |probability x value| per output, the size that rounding errors scale with."""
+    R, out, mag = H // Hkv, np.zeros(q.shape), np.zeros(q.shape)
+    mask = np.arange(pos0 + T)[None, :] > pos0 + np.arange(T)[:, None]
+    for b in range(B):
+        for h in range(H):
+            rows, cols = slice(h * dk, (h + 1) * dk), slice(b * T, (b + 1) * T)
+            g = slice(h // R * dk, (h // R + 1) * dk)
+            k, v = (c[b, :pos0 + T, g].astype(np.float64) for c in (kc, vc))
+            s = q[rows, cols].astype(np.float64).T @ k.T * scale
+            s[mask] = -np.inf
+            p = np.exp(s - s.max(1, keepdims=True))
+            p /= p.sum(1, keepdims=True)
+            out[rows, cols], mag[rows, cols] = (p @ v).T, (p @ np.abs(v)).T
+    return out, mag
+
+
+# value scales of (q, keys, values): ordinary, powers of two far apart, ends of the f16 halves' range,
+# and past it (f32 products)
+SCALES = [(1.0, 1.0, 1.0), (1e3, 1e-3, 1e-9), (1e-6, 1e6, 1e12), (1e-13, 1e13, 1.0), (1e20, 1e-20, 1e25), (1.0, 1.0, 1e-30)]
+
+
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("H,Hkv,dk,T,pos0", [(4, 4, 64, 257, 3), (4, 2, 128, 129, 31), (8, 1, 64, 33, 64), (4, 1, 128, 65, 0)])
+def test_prefill_halves_match_float64(ctx, H, Hkv, dk, T, pos0, f16):
+    """The f16-halves products at every group size, tails of queries and keys, values whose scale
+    rises and falls along the sequence, scores that keep growing, and scales past the halves' range:
+    within 1e-5 of float64 relative to sum |p v| (f32 scores of magnitude up to 25: 25 x 2^-24 each
+    in the exponent, and sums of at most 321 keys)."""
+    import torch
+    B, max_len = 2, pos0 + T + 3
+    scale = float(np.float32(1.0 / np.sqrt(dk)))
+    for i, (aq, ak, av) in enumerate(SCALES if not f16 else SCALES[:1]):
+        say(f"prefill halves H={H} Hkv={Hkv} dk={dk} T={T} pos0={pos0} f16={f16} scales={aq, ak, av}")
+        q = normal((H * dk, B * T), 900 + i) * np.float32(aq)
+        kc = normal((B, max_len, Hkv * dk), 910 + i) * np.float32(ak)
+        vc = normal((B, max_len, Hkv * dk), 920 + i) * np.float32(av)
+        ramp = np.linspace(0.2, 2.0, max_len, dtype=np.float32)[None, :, None]
+        kc = kc * ramp                                         # later keys score higher
+        vc = vc * np.exp2(np.round(6 * np.sin(np.arange(max_len) / 9.0))).astype(np.float32)[None, :, None]
+        cdt = np.float16 if f16 else np.float32
+        kc, vc = kc.astype(cdt), vc.astype(cdt)
+        got = host(ctx.attention_prefill(dev(q), dev(kc), dev(vc), B, T, H, Hkv, dk, pos0, scale))
+        ref, mag = attend64(q, kc, vc, B, T, H, Hkv, dk, pos0, float(np.float32(scale)))
+        err = np.abs(got.astype(np.float64) - ref) / np.maximum(mag, 1e-300)
+        assert float(err.max()) <= 1e-5, (aq, ak, av, float(err.max()))
+
+
+@pytest.mark.parametrize("f16", [False, True])
+def test_prefill_special_values(ctx, f16):
+    """A NaN or infinite key makes exactly the queries that see it NaN (+inf scores: inf - inf), a NaN
+    query its own head's column; a zero or negative scale and all-zero values are ordinary. The other
+    outputs stay within 1e-5 of float64 relative to sum |p v|."""
+    B, T, H, Hkv, dk, pos0 = 1, 150, 4, 2, 128, 10
+    max_len = pos0 + T
+    say(f"prefill special values f16={f16}")
+    cdt = np.float16 if f16 else np.float32
+    q = normal((H * dk, T), 940)
+    kc, vc = (normal((B, max_len, Hkv * dk), s).astype(cdt) for s in (941, 942))
+    scale = float(np.float32(1.0 / np.sqrt(dk)))
+
+    def close(got, ref, mag):
+        assert float((np.abs(got - ref) / np.maximum(mag, 1e-300)).max()) <= 1e-5
+
+    for bad in (np.nan, np.inf):
+        k2, q2 = kc.copy(), q.copy()
+        k2[0, pos0 + 70, 0:dk] = bad if np.isnan(bad) else 0.0
+        if np.isinf(bad):
+            k2[0, pos0 + 70, 5] = bad
+            q2[[5, dk + 5], 70:] = np.abs(q2[[5, dk + 5], 70:]) + 0.1   # +inf scores in the group's heads
+        q2[2 * dk + 7, 33] = np.nan                                    # one query of head 2
+        got = host(ctx.attention_prefill(dev(q2), dev(k2), dev(vc), B, T, H, Hkv, dk, pos0, scale)).astype(np.float64)
+        ref, mag = attend64(q2, kc, vc, B, T, H, Hkv, dk, pos0, scale)
+        nan = np.zeros(got.shape, bool)
+        nan[:2 * dk, 70:] = True
+        nan[2 * dk:3 * dk, 33] = True
+        assert np.array_equal(np.isnan(got), nan), bad
+        close(got[~nan], ref[~nan], mag[~nan])
+    for sc, v2 in ((0.0, vc), (-scale, vc), (scale, np.zeros_like(vc)), (1e-9, vc)):
+        got = host(ctx.attention_prefill(dev(q), dev(kc), dev(v2), B, T, H, Hkv, dk, pos0, sc)).astype(np.float64)
+        close(got, *attend64(q, kc, v2, B, T, H, Hkv, dk, pos0, float(np.float32(sc))))
