@@ -35,12 +35,13 @@
 // lane l holds query l % 32 throughout: its 16 elements v of S^T are keys 8(v/4) + 4(l/32) + v%4,
 // and V^T is staged with its keys in that order, so P^T is an operand as it stands. Row 32d + r of
 // V^T is dimension (DK/32) r + d, which lets a staging lane load contiguous dimensions and its
-// stores fall on all banks. K rows and V^T rows are XOR-swizzled in 16-byte chunks.
+// stores fall on all banks. K rows and V^T rows are padded to odd multiples of 16 bytes.
 // Softmax in log2 units with the hardware exp2; a query's reference maximum moves only when it has
 // grown by 2^8 (probabilities are held times 2^6, at most 2^14), so the sums are rarely rescaled.
 // Work-groups are issued heaviest first (the last query blocks attend over the most keys).
-// Measured (calls back to back, us, f32 products / here): f32 caches 4 x 2048 tokens 848 / 372,
-// 3 x 1111 at 517 432 / 186, 16 x 2048 3077 / 1242; f16 caches 821 / 235, 426 / 125, 3132 / 866.
+// Measured (calls back to back, us, f32 products / here): f32 caches 4 x 2048 tokens 848 / 328,
+// 3 x 1111 at 517 432 / 162, 16 x 2048 3077 / 1119, 1 x 64 21.9 / 13.9; f16 caches 821 / 209,
+// 426 / 105, 3132 / 774, 22.0 / 12.8.
 // Caches of f16 elements (compute = F16): the fill rounds the rotated keys and the values to the
 // nearest f16 (ties to even), as the decode append does.
 #include "common.hpp"
@@ -170,8 +171,12 @@ template <int DK, typename CT>
 struct PrefillTile
 {
     static constexpr int kPlanes = sizeof(CT) == 4 ? 2 : 1;  // high and low f16 halves of f32 values
-    static constexpr int kPlane = kPK * DK * 2;              // bytes of one plane of K or of V
-    static constexpr int kBuf = 2 * kPlanes * kPlane;        // K planes, then V planes
+    // rows are padded by 16 bytes: 16 lanes' reads of consecutive rows fall on all banks, and every
+    // chunk is at a constant offset from a lane's first
+    static constexpr int kKPitch = DK * 2 + 16, kVPitch = kPK * 2 + 16;
+    static constexpr int kKPlane = kPK * kKPitch, kVPlane = DK * kVPitch;
+    static constexpr int kV = kPlanes * kKPlane;             // K planes, then V planes
+    static constexpr int kBuf = kV + kPlanes * kVPlane;
     static constexpr int KROW = DK + 4;                      // f32 products: padded row (floats)
     static constexpr int kF32 = 2 * kPK * KROW * 4;
     static constexpr int kMain = 2 * kBuf > kF32 ? 2 * kBuf : kF32;  // double-buffered
@@ -182,8 +187,12 @@ struct PrefillTile
 __device__ __forceinline__ void split2(float x0, float x1, v2h& hi, v2h& lo)
 {
     hi = __builtin_convertvector(v2f{x0, x1}, v2h);
-    // one fma each: the differences are exact
-    lo = __builtin_convertvector(v2f{__builtin_fmaf((float)hi[0], -1.0f, x0), __builtin_fmaf((float)hi[1], -1.0f, x1)}, v2h);
+    // x - hi, exact, from the packed half in place (the compiler widens it with an instruction first)
+    const uint32_t u = __builtin_bit_cast(uint32_t, hi);
+    float l0, l1;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(l0) : "v"(u), "v"(x0));
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(l1) : "v"(u), "v"(x1));
+    lo = __builtin_convertvector(v2f{l0, l1}, v2h);
 }
 
 // 2^e for |e| <= 126
@@ -207,48 +216,53 @@ struct PrefillWave
     bool live;  // the wave has queries
 };
 
-// The lane's rotated query value pairs, f(dimension, value, value of dimension + DK/2) for its
-// dimensions below DK/2: those with (i / G) % 2 == h in groups of G
+// The lane's rotated query value pairs, f(c, e, value, value of the dimension DK/2 further) for its
+// dimensions 2Gc + Gh + e below DK/2. The cos / sin rows of 32 queries are 32 lines apart, so they
+// are read four at a time. Lanes past the last token repeat it (they are never stored).
 template <int DK, int G, typename F>
 __device__ __forceinline__ void load_query(const PrefillArgs& a, const PrefillWave& w, int h, F&& f)
 {
-    constexpr int HALF = DK / 2;
+    constexpr int HALF = DK / 2, NG = HALF / (2 * G);
     const int M = a.B * a.T;
     const __amdgpu_buffer_rsrc_t rq = pf_rsrc(a.q, (uint32_t)((size_t)a.H * DK * (size_t)M * 4u));
-    const __amdgpu_buffer_rsrc_t rc = pf_rsrc(a.cosT ? a.cosT : a.q, a.cosT ? (uint32_t)((size_t)a.max_len * HALF * 4u) : 0u);
-    const __amdgpu_buffer_rsrc_t rs = pf_rsrc(a.cosT ? a.sinT : a.q, a.cosT ? (uint32_t)((size_t)a.max_len * HALF * 4u) : 0u);
-    const bool qok = w.qt < a.T;
-    const int m = w.b * a.T + w.qt;
+    const uint32_t rope_bytes = a.cosT ? (uint32_t)((size_t)a.max_len * HALF * 4u) : 0u;
+    const __amdgpu_buffer_rsrc_t rc = pf_rsrc(a.cosT ? a.cosT : a.q, rope_bytes);
+    const __amdgpu_buffer_rsrc_t rs = pf_rsrc(a.cosT ? a.sinT : a.q, rope_bytes);
+    const int qt = min(w.qt, a.T - 1);
+    const uint32_t q_at = (uint32_t)(((size_t)(w.head * DK + G * h) * (size_t)M + (size_t)(w.b * a.T + qt)) * 4u);
+    const uint32_t r_at = (uint32_t)(((size_t)(a.pos0 + qt) * HALF + (size_t)(G * h)) * 4u);
 #pragma unroll
-    for (int c = 0; c < HALF / (2 * G); ++c)
+    for (int c = 0; c < NG; ++c)
     {
-        float x0[G], x1[G], cs[G], sn[G];
+        float x[2][G];
+        float4 cs[G / 4], sn[G / 4];
 #pragma unroll
         for (int e = 0; e < G; ++e)
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+                x[q][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rq, q_at, (2 * G * c + e + HALF * q) * M * 4, 0));
+#pragma unroll
+        for (int e = 0; e < G / 4; ++e)
         {
-            const int i = 2 * G * c + G * h + e;
-            const size_t at = ((size_t)(w.head * DK + i) * (size_t)M + (size_t)m) * 4u;
-            x0[e] = ld_f(rq, qok ? (uint32_t)at : 0x80000000u);
-            x1[e] = ld_f(rq, qok ? (uint32_t)(at + (size_t)HALF * (size_t)M * 4u) : 0x80000000u);
-            const uint32_t off = qok ? (uint32_t)(((size_t)w.qpos * HALF + (size_t)i) * 4u) : 0x80000000u;
-            cs[e] = ld_f(rc, off);
-            sn[e] = ld_f(rs, off);
+            cs[e] = ld_f4(rc, r_at + (uint32_t)(2 * G * c + 4 * e) * 4u);
+            sn[e] = ld_f4(rs, r_at + (uint32_t)(2 * G * c + 4 * e) * 4u);
         }
 #pragma unroll
         for (int e = 0; e < G; ++e)
         {
-            float y0 = x0[e], y1 = x1[e];
-            if (a.cosT) pf_rope(x0[e], x1[e], cs[e], sn[e], y0, y1);
+            const float cv = e % 4 == 0 ? cs[e / 4].x : e % 4 == 1 ? cs[e / 4].y : e % 4 == 2 ? cs[e / 4].z : cs[e / 4].w;
+            const float sv = e % 4 == 0 ? sn[e / 4].x : e % 4 == 1 ? sn[e / 4].y : e % 4 == 2 ? sn[e / 4].z : sn[e / 4].w;
+            float y0 = x[0][e], y1 = x[1][e];
+            if (a.cosT) pf_rope(x[0][e], x[1][e], cv, sv, y0, y1);
             f(c, e, y0, y1);
         }
     }
 }
 
-// out[head*DK + i][m] for the lane's query: element v of block d belongs to row r = 8(v/4) + 4h + v%4
-// of the block; dim(d, r) is its dimension
-template <int DK, typename D>
-__device__ __forceinline__ void store_out(const PrefillArgs& a, const PrefillWave& w, const v16f* o, float l, int e, int h,
-                                          D&& dim)
+// out[head*DK + i][m] = y(d, v) for the lane's query: element v of block d belongs to row
+// r = 8(v/4) + 4h + v%4 of the block; dim(d, r) is its dimension
+template <int DK, typename D, typename Y>
+__device__ __forceinline__ void store_out(const PrefillArgs& a, const PrefillWave& w, int h, D&& dim, Y&& y)
 {
     if (w.qt >= a.T) return;
     const int M = a.B * a.T, m = w.b * a.T + w.qt;
@@ -256,8 +270,7 @@ __device__ __forceinline__ void store_out(const PrefillArgs& a, const PrefillWav
     for (int d = 0; d < DK / 32; ++d)
 #pragma unroll
         for (int v = 0; v < 16; ++v)
-            a.out[(size_t)(w.head * DK + dim(d, 8 * (v >> 2) + 4 * h + (v & 3))) * (size_t)M + (size_t)m] =
-                ldexpf(o[d][v] / l, -e);
+            a.out[(size_t)(w.head * DK + dim(d, 8 * (v >> 2) + 4 * h + (v & 3))) * (size_t)M + (size_t)m] = y(d, v);
 }
 
 // The work-group's attention on the fp32 MFMA (v_mfma_f32_32x32x2_f32), for inputs that the f16
@@ -346,7 +359,8 @@ __device__ void attend_f32(const PrefillArgs& a, const PrefillWave& w, int last_
                 o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(vs[key * KROW + 32 * d + l32], sc[sp], o[d], 0, 0, 0);
             }
     }
-    if (w.live) store_out<DK>(a, w, o, l_run, 0, h, [](int d, int r) { return 32 * d + r; });
+    if (w.live)
+        store_out<DK>(a, w, h, [](int d, int r) { return 32 * d + r; }, [&](int d, int v) { return o[d][v] / l_run; });
 }
 
 template <int DK, typename CT>
@@ -400,69 +414,69 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
     const bool is_v = wave < 4;
     const int u = tid & 255;
     const int vq = u >> 5, vg = u & 31;  // V: key quad, dimension group
+    // the thread's offsets within a tile; the tile's rows are reached through the buffer's base
+    constexpr int NL = F32C ? 4 : (4 > KU ? 4 : KU);
+    uint32_t at[NL];
+#pragma unroll
+    for (int i = 0; i < NL; ++i)
+    {
+        const int ct = u + 256 * i;
+        at[i] = is_v ? (uint32_t)(((4 * vq + i) * row + w.g * DK + ND * vg) * (int)sizeof(CT))
+                     : (uint32_t)((ct / CH * row + w.g * DK + 8 * (ct % CH)) * (int)sizeof(CT));
+    }
+    const uint32_t tile_bytes = (uint32_t)(kPK * row) * (uint32_t)sizeof(CT);
+    const CT* const kvb = (is_v ? static_cast<const CT*>(a.vc) : static_cast<const CT*>(a.kc)) + seq_off;
     auto load_raw = [&](int kb) {
+        const uint64_t before = (uint64_t)kb * tile_bytes;
+        const __amdgpu_buffer_rsrc_t rt = pf_rsrc(reinterpret_cast<const uint8_t*>(kvb) + before,
+                                                  before < seq_bytes ? seq_bytes - (uint32_t)before : 0u);
         if (is_v)
         {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
             {
-                const uint32_t off = (uint32_t)(((size_t)(kb * kPK + 4 * vq + i) * (size_t)row + (size_t)w.g * DK + ND * vg) * sizeof(CT));
                 constexpr int W = ND * (int)sizeof(CT) / 4;  // words per key
                 if constexpr (W == 4)
                 {
-                    const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(rv, off, 0, 0);
+                    const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(rt, at[i], 0, 0);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) raw[4 * i + e] = x[e];
                 }
                 else if constexpr (W == 2)
                 {
                     typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-                    const u32x2 x = __builtin_amdgcn_raw_buffer_load_b64(rv, off, 0, 0);
+                    const u32x2 x = __builtin_amdgcn_raw_buffer_load_b64(rt, at[i], 0, 0);
                     raw[2 * i] = x[0];
                     raw[2 * i + 1] = x[1];
                 }
-                else raw[i] = __builtin_amdgcn_raw_buffer_load_b32(rv, off, 0, 0);
+                else raw[i] = __builtin_amdgcn_raw_buffer_load_b32(rt, at[i], 0, 0);
             }
         }
         else
         {
 #pragma unroll
             for (int j = 0; j < KU; ++j)
-            {
-                const int ct = u + 256 * j;
-                const uint32_t off = (uint32_t)(((size_t)(kb * kPK + ct / CH) * (size_t)row + (size_t)w.g * DK + 8 * (ct % CH)) * sizeof(CT));
 #pragma unroll
                 for (int q = 0; q < (F32C ? 2 : 1); ++q)
                 {
-                    const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(rk, off + 16 * q, 0, 0);
+                    const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(rt, at[j] + 16 * q, 0, 0);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) raw[(F32C ? 8 : 4) * j + 4 * q + e] = x[e];
                 }
-            }
         }
     };
     // words of raw in use
     constexpr int VW = 4 * ND * (int)sizeof(CT) / 4, KW = KU * 8 * (int)sizeof(CT) / 4;
     static_assert(VW == KW && VW <= RW, "V and K threads stage the same amount");
-    // f32: the wave's largest magnitude for the tile's scaling; f16: only whether all are finite
-    auto post_max = [&](int kb, int* flag) {
-        uint32_t mx = 0;
+    // f32 caches: the wave's largest magnitude, for the tile's scaling
+    auto post_max = [&](int kb) {
         if constexpr (F32C)
         {
+            uint32_t mx = 0;
 #pragma unroll
             for (int e = 0; e < VW; ++e) mx = max(mx, raw[e] & 0x7FFFFFFFu);
             mx = wave_max(mx);
             if (lane == 0) smax[(kb & 1) * 8 + wave] = mx;
-        }
-        else
-        {
-#pragma unroll
-            for (int e = 0; e < VW; ++e)
-            {
-                mx = max(mx, raw[e] & 0x7FFFu);
-                mx = max(mx, (raw[e] >> 16) & 0x7FFFu);
-            }
-            if (__builtin_amdgcn_ballot_w64(mx >= 0x7C00u) != 0 && lane == 0) *flag = 1;
         }
     };
     int ek = 0, ev = 1 << 20;  // exponents of the staged tile: K's own, V's running smallest
@@ -492,7 +506,7 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
             for (int e = 0; e < ND; ++e)
             {
                 const int r = 32 * e + vg;
-                uint8_t* dst = buf + Tile::kPlanes * Tile::kPlane + r * 64 + (((2 * s + hh) ^ ((r >> 2) & 3)) << 4) + 8 * ah;
+                uint8_t* dst = buf + Tile::kV + r * Tile::kVPitch + 32 * s + 16 * hh + 8 * ah;
                 if constexpr (F32C)
                 {
                     float x[4];
@@ -502,7 +516,7 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
                     split2(x[0], x[1], h0, l0);
                     split2(x[2], x[3], h1, l1);
                     *reinterpret_cast<v4h*>(dst) = v4h{h0[0], h0[1], h1[0], h1[1]};
-                    *reinterpret_cast<v4h*>(dst + Tile::kPlane) = v4h{l0[0], l0[1], l1[0], l1[1]};
+                    *reinterpret_cast<v4h*>(dst + Tile::kVPlane) = v4h{l0[0], l0[1], l1[0], l1[1]};
                 }
                 else
                 {
@@ -521,7 +535,7 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
             for (int j = 0; j < KU; ++j)
             {
                 const int ct = u + 256 * j, key = ct / CH, c = ct % CH;
-                uint8_t* dst = buf + key * DK * 2 + ((c ^ (CH == 16 ? key & 15 : (key >> 1) & 7)) << 4);
+                uint8_t* dst = buf + key * Tile::kKPitch + 16 * c;
                 if constexpr (F32C)
                 {
                     v8h hi, lo;
@@ -534,7 +548,7 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
                         lo[e] = y[0], lo[e + 1] = y[1];
                     }
                     *reinterpret_cast<v8h*>(dst) = hi;
-                    *reinterpret_cast<v8h*>(dst + Tile::kPlane) = lo;
+                    *reinterpret_cast<v8h*>(dst + Tile::kKPlane) = lo;
                 }
                 else
                     *reinterpret_cast<u32x4*>(dst) = u32x4{raw[4 * j], raw[4 * j + 1], raw[4 * j + 2], raw[4 * j + 3]};
@@ -544,31 +558,27 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
 
     // Fragments from LDS, four 16-byte reads at a time, a group ahead of the products that use them:
     // group g of K holds steps GS g .., group g of V^T (block, half) pairs GS g .., each with its low
-    // plane next to it for f32 caches. The chunk swizzles are XORs of address bits that no other term
-    // of the offset reaches.
+    // plane next to it for f32 caches.
     constexpr int GS = 4 / Tile::kPlanes;
     static_assert(NC % GS == 0 && (2 * ND) % GS == 0, "whole groups");
-    const uint32_t k_at = (uint32_t)(l32 * DK * 2 + ((h ^ (CH == 16 ? l32 & 15 : (l32 >> 1) & 7)) << 4));
-    const uint32_t v_at = (uint32_t)(Tile::kPlanes * Tile::kPlane + l32 * 64 + ((h ^ ((l32 >> 2) & 3)) << 4));
+    const uint32_t k_at = (uint32_t)(l32 * Tile::kKPitch + 16 * h), v_at = (uint32_t)(Tile::kV + l32 * Tile::kVPitch + 16 * h);
     auto read_k = [&](v8h(&f)[4], uint32_t par, int g) {
+        const uint8_t* p = smem + (par + k_at);
 #pragma unroll
         for (int e = 0; e < GS; ++e)
-        {
-            const uint8_t* p = smem + ((par + k_at) ^ (uint32_t)((GS * g + e) << 5));
 #pragma unroll
             for (int q = 0; q < Tile::kPlanes; ++q)
-                f[Tile::kPlanes * e + q] = *reinterpret_cast<const v8h*>(p + q * Tile::kPlane);
-        }
+                f[Tile::kPlanes * e + q] = *reinterpret_cast<const v8h*>(p + 32 * (GS * g + e) + q * Tile::kKPlane);
     };
     auto read_v = [&](v8h(&f)[4], uint32_t par, int g) {
+        const uint8_t* p = smem + (par + v_at);
 #pragma unroll
         for (int e = 0; e < GS; ++e)
         {
             const int d = (GS * g + e) >> 1, t = (GS * g + e) & 1;
-            const uint8_t* p = smem + ((par + v_at) ^ (uint32_t)(t << 5)) + d * 2048;
 #pragma unroll
             for (int q = 0; q < Tile::kPlanes; ++q)
-                f[Tile::kPlanes * e + q] = *reinterpret_cast<const v8h*>(p + q * Tile::kPlane);
+                f[Tile::kPlanes * e + q] = *reinterpret_cast<const v8h*>(p + 32 * d * Tile::kVPitch + 32 * t + q * Tile::kVPlane);
         }
     };
 
@@ -611,13 +621,13 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
     float m_ref = -__builtin_inff(), l_run = 0.0f;  // log2 units; l_run: this lane half's keys
     int eo = 0;                                     // the exponent of V in o
 
-    post_max(0, sflag);
+    post_max(0);
     __syncthreads();
     convert(0, sflag);
     if (nkb > 1)
     {
         load_raw(1);
-        post_max(1, sflag);
+        post_max(1);
     }
     bool fallback = false;
     for (int kb = 0; kb < nkb; ++kb)
@@ -726,7 +736,17 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        if (kb + 2 < nkb) post_max(kb + 2, sflag + ((kb + 1) & 1));
+        if (kb + 2 < nkb) post_max(kb + 2);
+    }
+    if constexpr (!F32C)
+    {
+        // f16 caches are not looked through for infinities and NaN: any that matters is in the sums
+        bool bad = !(fabsf(l_run) < __builtin_inff());
+#pragma unroll
+        for (int d = 0; d < ND; ++d)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) bad |= !(fabsf(o[d][v]) < __builtin_inff());
+        fallback = __syncthreads_or(!fallback && w.live && bad) || fallback;
     }
     if (fallback)
     {
@@ -734,8 +754,14 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
         return;
     }
     l_run += __shfl_xor(l_run, 32);
-    if (w.live)
-        store_out<DK>(a, w, o, l_run, F32C ? eo : 0, h, [](int d, int r) { return ND * r + d; });
+    if (!w.live) return;
+    // o / l (correctly rounded but for the last step's double rounding: the residual is exact) and
+    // V's exponent back; an all-zero V has none
+    const float r = 1.0f / l_run, back = F32C ? pow2(eo > kPExpMax ? 0 : -eo) : 1.0f;
+    store_out<DK>(a, w, h, [](int d, int i) { return ND * i + d; }, [&](int d, int v) {
+        const float q = o[d][v] * r, y = __builtin_fmaf(__builtin_fmaf(-q, l_run, o[d][v]), r, q);
+        return F32C ? y * back : y;
+    });
 }
 
 template <int DK, typename CT>
