@@ -684,6 +684,41 @@ __global__ __launch_bounds__(kSmallBlock) void k_embed(const float* __restrict__
     out[tm ? (size_t)b * d + i : (size_t)i * B + b] = (id >= 0 && id < V) ? table[(size_t)id * d + i] : __builtin_nanf("");
 }
 
+// out (d, B) for many tokens: block = 64 tokens x 64 features, the table rows read along features
+// and the columns written along tokens through LDS. Bound by HBM (4dB bytes read and written); one
+// element per thread as above stores 64 separate lines per instruction: 2560 x 8192 tokens
+// 166.7 -> 25.3 us (6.6 TB/s), 1024 tokens 17.4 -> 5.3 us.
+constexpr int kEmbTile = 64;
+
+__global__ __launch_bounds__(kSmallBlock) void k_embed_cols(const float* __restrict__ table, const int32_t* __restrict__ ids,
+                                                            int V, int d, int B, float* __restrict__ out)
+{
+    constexpr int NW = kSmallBlock / kWave, N = kEmbTile / NW;
+    __shared__ float tile[kEmbTile][kEmbTile + 1];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int b0 = blockIdx.x * kEmbTile, f0 = blockIdx.y * kEmbTile;
+    const int idv = ids[min(b0 + lane, B - 1)];
+    const int f = min(f0 + lane, d - 1);  // loads past the ends repeat the last token or feature
+    float x[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+    {
+        const int id = __builtin_amdgcn_readlane(idv, NW * i + w);
+        const bool ok = id >= 0 && id < V;
+        const float v = table[(size_t)(ok ? id : 0) * d + f];
+        x[i] = ok ? v : __builtin_nanf("");
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) tile[NW * i + w][lane] = x[i];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+    {
+        const int r = NW * i + w;
+        if (f0 + r < d && b0 + lane < B) out[(size_t)(f0 + r) * B + b0 + lane] = tile[lane][r];
+    }
+}
+
 // ids[b] = the reference greedy rule over column b of logits (V, B): best = l[0], then every
 // l[v] > best replaces it (first index of the largest value; NaN entries never win, a NaN at
 // v = 0 keeps index 0).
@@ -805,6 +840,14 @@ hipError_t launch_copy_cols(hipStream_t st, const float* src, size_t rows, size_
 hipError_t launch_embed(hipStream_t st, const float* table, const int32_t* ids, size_t V, size_t d, size_t B, bool tm,
                         float* out)
 {
+    // below a tile of tokens the scattered stores are few (48 tokens 3.0 against 3.3 us, 64 3.3 both,
+    // 128 4.4 against 3.4)
+    if (!tm && B >= kEmbTile)
+    {
+        k_embed_cols<<<dim3((unsigned)ceil_div(B, kEmbTile), (unsigned)ceil_div(d, kEmbTile)), kSmallBlock, 0, st>>>(
+            table, ids, (int)V, (int)d, (int)B, out);
+        return hipGetLastError();
+    }
     k_embed<<<dim3((unsigned)ceil_div(d, kSmallBlock), (unsigned)B), kSmallBlock, 0, st>>>(table, ids, (int)V, (int)d,
                                                                                          (int)B, tm ? 1 : 0, out);
     return hipGetLastError();

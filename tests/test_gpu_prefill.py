@@ -437,3 +437,14 @@ def test_prefill_special_values(ctx, f16):
     for sc, v2 in ((0.0, vc), (-scale, vc), (scale, np.zeros_like(vc)), (1e-9, vc)):
         got = host(ctx.attention_prefill(dev(q), dev(kc), dev(v2), B, T, H, Hkv, dk, pos0, sc)).astype(np.float64)
         close(got, *attend64(q, kc, v2, B, T, H, Hkv, dk, pos0, float(np.float32(sc))))
+
+
+@pytest.mark.parametrize("V,d,B", [(50, 64, 64), (97, 300, 129), (1000, 2560, 1000), (7, 1, 65)])
+def test_embedding_gather_many_tokens(ctx, V, d, B):
+    """Tiles of 64 tokens and 64 features with tails of both, ids outside the table as NaN columns."""
+    import torch
+    table, ids = normal((V, d), 950 + d), (np.arange(B, dtype=np.int64) * 7919 % V).astype(np.int32)
+    ids[[3, B - 1]] = -1, V
+    ref = table[np.clip(ids, 0, V - 1)].T.copy()
+    ref[:, [3, B - 1]] = np.nan
+    assert same_bits(host(ctx.embedding_gather(dev(table), dev(ids))), ref)
