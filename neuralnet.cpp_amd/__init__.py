@@ -245,6 +245,11 @@ class Context:
         if not torch.cuda.is_available():
             raise NNHipError(4, "no GPU visible to torch")
         self.device = device
+        self._device = torch.device("cuda", device)
+        # the current stream's handle without a Stream object around it (0.1 instead of 1.1 us; a
+        # call's Python side is on the critical path of a decode-size kernel)
+        self._raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or \
+            (lambda d: torch.cuda.current_stream(d).cuda_stream)
         h = _vp()
         _check(lib().nnhip_ctx_create(device, ctypes.byref(h)), "nnhip_ctx_create")
         self.h = h
@@ -262,23 +267,24 @@ class Context:
 
     # -- helpers
     def _bind_stream(self) -> None:
-        s = self._torch.cuda.current_stream(self.device).cuda_stream
-        _check(lib().nnhip_ctx_set_stream(self.h, _vp(s)), "nnhip_ctx_set_stream")
+        st = lib().nnhip_ctx_set_stream(self.h, self._raw_stream(self.device))
+        if st != 0:
+            _check(st, "nnhip_ctx_set_stream")
 
     def _dev(self, t, dtype=None, name="tensor"):
-        torch = self._torch
+        """The device address of t (None: null), after its checks."""
         if t is None:
             return None
         if not t.is_cuda:
             raise NNHipError(1, f"{name} must be a device tensor")
         if not t.is_contiguous():
             raise NNHipError(1, f"{name} must be contiguous")
-        if dtype is not None and t.dtype not in (dtype if isinstance(dtype, tuple) else (dtype,)):
+        if dtype is not None and t.dtype is not dtype and t.dtype not in (dtype if isinstance(dtype, tuple) else (dtype,)):
             raise NNHipError(1, f"{name} has dtype {t.dtype}, expected {dtype}")
-        return _vp(t.data_ptr())
+        return t.data_ptr()
 
     def _empty(self, shape, dtype):
-        return self._torch.empty(shape, dtype=dtype, device=f"cuda:{self.device}")
+        return self._torch.empty(shape, dtype=dtype, device=self._device)
 
     def sync(self) -> None:
         self._bind_stream()
