@@ -275,9 +275,20 @@ hipError_t launch_gemv_grouped(hipStream_t st, const GemvProblem* d_probs, const
                                const uint32_t* d_wave_items, size_t n_waves, const XStage* d_xstage,
                                int n_xstage, uint32_t lds_bytes);
 size_t gemv_grid_waves(size_t n_items, int num_cus, bool lds);
-// Prefill GEMM; tile is one of NNHIP_GEMM_TILE_* (AUTO: gemm_tile_choice).
+// Prefill GEMM; tile is one of NNHIP_GEMM_TILE_* (AUTO: skinny_plan, else gemm_split_choice).
 hipError_t launch_gemm(hipStream_t st, const GemvProblem& p, int num_cus, int tile);
 hipError_t launch_gemm_digits(hipStream_t st, const GemvProblem& p, const DigitOut& g, int num_cus, int tile);
+
+// ---- products between the decode GEMV and the prefill GEMM (k_skinny.hip); waves == 0: the GEMM
+struct SkinnyPlan
+{
+    int row_tiles;  // 16-row tiles per block
+    int groups;     // 16-token groups per block
+    int mblocks;    // blocks over the tokens
+    int waves;      // waves per block, splitting the reduction
+};
+SkinnyPlan skinny_plan(const GemvProblem& p, int num_cus, double gemm_rounds);
+hipError_t launch_skinny(hipStream_t st, const GemvProblem& p, const DigitOut* dg, const SkinnyPlan& s);
 int gemm_tile_choice(const GemvProblem& p, int num_cus);
 // Time of one round of 128 x 128 / 64 x 64 blocks relative to one round of 256 x 128 blocks,
 // measured over M = 128..4096, K = 2560..6912, N = 2560..13824 (with these the automatic choice
@@ -290,6 +301,7 @@ constexpr double kGemmRelB = 0.6, kGemmRelC = 0.45;
 struct GemmSplit
 {
     int tile, rows, tail_tile;
+    double rounds;  // estimated 256 x 128 rounds of the choice
 };
 constexpr double kGemmSplitCost = 0.1;
 GemmSplit gemm_split_choice(const GemvProblem& p, int num_cus);

@@ -943,23 +943,24 @@ GemvProblem gemm_rows_from(const GemvProblem& p, int rows0)
 
 GemmSplit gemm_split_choice(const GemvProblem& p, int num_cus)
 {
-    GemmSplit s{gemm_tile_choice(p, num_cus), 0, 0};
+    GemmSplit s{gemm_tile_choice(p, num_cus), 0, 0, 0.0};
     const int cus = num_cus > 0 ? num_cus : 256;
     const int n_mb = (int)ceil_div((size_t)p.M, (size_t)GemmA::kBM);
     const int n_nb = (int)ceil_div((size_t)p.N, (size_t)GemmA::kBN);
     // the longest row-block prefix whose 256 x 128 blocks fill whole rounds of the CUs
     int r1 = n_nb - 1;
     while (r1 > 0 && ((long)r1 * n_mb) % cus != 0) --r1;
-    if (r1 <= 0) return s;
     const double best = s.tile == NNHIP_GEMM_TILE_256x128   ? gemm_cost(p, cus, GemmA::kBN, GemmA::kBM, 1.0)
                         : s.tile == NNHIP_GEMM_TILE_128x128 ? gemm_cost(p, cus, GemmB::kBN, GemmB::kBM, kGemmRelB)
                                                             : gemm_cost(p, cus, GemmC::kBN, GemmC::kBM, kGemmRelC);
+    s.rounds = best;
+    if (r1 <= 0) return s;
     const GemvProblem tail = gemm_rows_from(p, r1 * GemmA::kBN);
     const double tb = gemm_cost(tail, cus, GemmB::kBN, GemmB::kBM, kGemmRelB);
     const double tc = gemm_cost(tail, cus, GemmC::kBN, GemmC::kBM, kGemmRelC);
     const double split = (double)((long)r1 * n_mb / cus) + (tb <= tc ? tb : tc) + kGemmSplitCost;
     if (split < best) s = GemmSplit{NNHIP_GEMM_TILE_256x128, r1 * GemmA::kBN,
-                                    tb <= tc ? NNHIP_GEMM_TILE_128x128 : NNHIP_GEMM_TILE_64x64};
+                                    tb <= tc ? NNHIP_GEMM_TILE_128x128 : NNHIP_GEMM_TILE_64x64, split};
     return s;
 }
 
@@ -980,6 +981,8 @@ hipError_t launch_any(hipStream_t st, const GemvProblem& p, int num_cus, int til
     if (tile == NNHIP_GEMM_TILE_AUTO)
     {
         const GemmSplit s = gemm_split_choice(p, num_cus);
+        const SkinnyPlan sk = skinny_plan(p, num_cus, s.rounds);
+        if (sk.waves > 0) return launch_skinny(st, p, dig, sk);
         if (s.rows > 0)
         {
             GemvProblem head = p, tail = gemm_rows_from(p, s.rows);

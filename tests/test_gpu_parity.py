@@ -741,3 +741,71 @@ def test_stream_xor(ctx, nbytes):
     assert got == int(np.bitwise_xor.reduce(words))
     ctx.stream_xor(src, out)
     assert int(out.cpu().numpy().view(np.uint32)[0]) == 0
+
+
+# block shapes of the split-reduction kernel between the GEMV and the GEMM (row tiles x token groups 1 x 1,
+# 2 x 1, 4 x 1, 4 x 2), with tails of rows, tokens and k, one k tile (idle waves) and many
+SKINNY = [(300, 520, 17), (2551, 1000, 40), (2575, 2560, 63), (2575, 700, 190), (100, 16, 33), (640, 7000, 129),
+          (5000, 257, 50)]
+
+
+@pytest.mark.parametrize("N,K,M", SKINNY)
+def test_between_gemv_and_gemm_bits(ctx, orc, N, K, M):
+    """17 to a few hundred tokens: every output equals the 64 x 64 GEMM tile's bit for bit (integer sums,
+    one epilogue), with bias and residual, and on a sample of tokens the oracle's."""
+    import torch
+    say(f"between GEMV and GEMM N={N} K={K} M={M}")
+    W, X = normal((N, K), N + K, 0.0, 0.02), normal((K, M), N + M)
+    tau = np.abs(W.astype(np.float64)).mean(axis=1).astype(np.float32)
+    bias = torch.from_numpy(normal((N,), M)).cuda()
+    res = torch.from_numpy(normal((N, M), 3 + M)).cuda()
+    wq = orc.trit_pack(W, tau)
+    rp, td = ctx.repack(torch.from_numpy(wq.view(np.int32)).cuda(), K), torch.from_numpy(tau).cuda()
+    acts = ctx.act_quant_i8(torch.from_numpy(X).cuda())
+    calls = [lambda: ctx.ternary_matmul(rp, td, *acts, N, K, M),
+             lambda: ctx.ternary_matmul(rp, td, *acts, N, K, M, bias=bias),
+             lambda: ctx.ternary_matmul_add(rp, td, *acts, N, K, M, res, bias=bias)]
+    got = [f() for f in calls]
+    ctx.set_gemm_tile(3)
+    try:
+        for g, f in zip(got, calls):
+            assert torch.equal(g.view(torch.int32), f().view(torch.int32))
+    finally:
+        ctx.set_gemm_tile(0)
+    s = orc.act_scale(X)
+    ref = orc.matmul_q_i8(wq, tau, orc.quantize_i8(X, s, True), s, K, M)
+    assert np.array_equal(got[0].cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("N,K,M", SKINNY)
+def test_between_gemv_and_gemm_gated_and_digits(ctx, orc, N, K, M):
+    """The gated epilogue (F = N / 2 features, not a multiple of 8) and the digit products of float
+    activations (M / 4 tokens, one of them special) on the same shapes, against the GEMM tile's bits."""
+    import torch
+    F = N // 2
+    say(f"between GEMV and GEMM, gated and digits F={F} K={K} M={M}")
+    W1 = torch.from_numpy(normal((2 * F, K), N + 2 * K, 0.0, 0.02)).cuda()
+    t1 = ctx.row_absmean(W1)
+    b1 = torch.from_numpy(normal((2 * F,), K)).cuda()
+    wo, to, bo = ctx.glu_interleave(ctx.trit_pack(W1, t1), t1, b1, F, K)
+    rp1 = ctx.repack(wo, K)
+    X = torch.from_numpy(normal((K, M), N + M)).cuda()
+    acts = ctx.act_quant_i8(X)
+    Mf = (M + 3) // 4 + 4
+    Xf = torch.from_numpy(normal((K, Mf), 5 + M)).cuda()
+    Xf[0, 2] = float("nan")
+    rpf = ctx.repack(ctx.trit_pack(W1, t1), K)
+    calls = [lambda: ctx.ternary_matmul_glu(rp1, to, *acts, F, K, M, 0, bias=bo),
+             lambda: ctx.ternary_matmul_glu(rp1, to, *acts, F, K, M, 1),
+             lambda: ctx.ternary_matmul_f(rpf, t1, Xf, 2 * F, K),
+             lambda: ctx.ternary_matmul_f(rpf, t1, Xf, 2 * F, K, out_f16=True).view(torch.int16)]
+    got = [f() for f in calls]
+    ctx.set_gemm_tile(3)
+    try:
+        for g, f in zip(got, calls):
+            r = f()
+            assert torch.equal(torch.isnan(g), torch.isnan(r)) if g.is_floating_point() else True
+            assert torch.equal(torch.nan_to_num(g) if g.is_floating_point() else g,
+                               torch.nan_to_num(r) if r.is_floating_point() else r)
+    finally:
+        ctx.set_gemm_tile(0)
