@@ -289,6 +289,9 @@ struct SkinnyPlan
 };
 SkinnyPlan skinny_plan(const GemvProblem& p, int num_cus, double gemm_rounds);
 hipError_t launch_skinny(hipStream_t st, const GemvProblem& p, const DigitOut* dg, const SkinnyPlan& s);
+// the same kernel for M <= 16 (residual and gated epilogue included) where it is the faster one
+bool gemv_split_ok(const GemvProblem& p, int num_cus);
+hipError_t launch_gemv_split(hipStream_t st, const GemvProblem& p, int num_cus);
 int gemm_tile_choice(const GemvProblem& p, int num_cus);
 // Time of one round of 128 x 128 / 64 x 64 blocks relative to one round of 256 x 128 blocks,
 // measured over M = 128..4096, K = 2560..6912, N = 2560..13824 (with these the automatic choice

@@ -1,5 +1,6 @@
 // k_skinny.hip — ternary x int8 products of 17 to a few hundred tokens on gfx950 int8 MFMA, between
-// the decode GEMV (k_gemv.hip, M <= 16) and the prefill GEMM (k_gemm.hip).
+// the decode GEMV (k_gemv.hip, M <= 16) and the prefill GEMM (k_gemm.hip), and of fewer tokens on the
+// shapes that the decode GEMV is not built for.
 //
 // There the GEMM's 64 x 64 blocks are few (40 for 2560 rows and up to 64 tokens, of 256 CUs) and each
 // walks the whole reduction stage by stage, so its time is a chain of K / 256 memory latencies: 8 us
@@ -228,6 +229,25 @@ hipError_t launch_skinny(hipStream_t st, const GemvProblem& p, const DigitOut* d
     if (dg) return launch_skinny_mode<kSkDigits>(st, p, *dg, s);
     if (p.glu) return launch_skinny_mode<kSkGlu>(st, p, none, s);
     return launch_skinny_mode<kSkPlain>(st, p, none, s);
+}
+
+// M <= 16: the shapes the deep GEMV is not built for, but for the ones the streaming GEMV has waves
+// and LDS for (more than 4 row tiles per CU, activations within its budget: 2560 -> 60000 at 16 tokens
+// 9.0 against 10.6 us). Elsewhere that kernel walks the k tiles in turn: 5120 -> 3000 at 1 / 16 tokens
+// 7.1 / 24.7 -> 3.4 / 4.8 us, 11008 -> 4096 13.4 / 44.3 -> 4.4 / 8.0, 12000 -> 16000 16.7 / 49.2 ->
+// 9.6 / 11.1. The deep GEMV's own shapes stay with it: in a decode step, whose weights come from HBM,
+// 552 against 560 us with this kernel in its place.
+bool gemv_split_ok(const GemvProblem& p, int num_cus)
+{
+    if (p.M < 1 || p.M > kGemvMaxM || p.ytm || gemv_deep_ok(p, num_cus)) return false;
+    const bool streams = (uint32_t)p.M * (uint32_t)p.KT * kTileK <= kGemvLdsBudget &&
+                         (p.N + 15) / 16 > kGemvDeepMaxTilesPerCu * (num_cus > 0 ? num_cus : 256);
+    return !streams;
+}
+
+hipError_t launch_gemv_split(hipStream_t st, const GemvProblem& p, int num_cus)
+{
+    return launch_skinny(st, p, nullptr, skinny_plan(p, num_cus, 1e300));
 }
 
 }  // namespace nnhip

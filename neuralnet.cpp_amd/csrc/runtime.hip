@@ -219,6 +219,12 @@ nnhip_status run_matmul(nnhip_ctx* ctx, const char* fn, const void* rp, const fl
         NNHIP_LAUNCH(fn, launch_gemv_deep(ctx->stream, p));
         return NNHIP_OK;
     }
+    if (M <= (size_t)kGemvMaxM && gemv_split_ok(p, ctx->num_cus))
+    {
+        p.res = res;
+        NNHIP_LAUNCH(fn, launch_gemv_split(ctx->stream, p, ctx->num_cus));
+        return NNHIP_OK;
+    }
     if (M <= (size_t)kGemvMaxM)
         NNHIP_LAUNCH(fn, launch_gemv(ctx->stream, p, ctx->num_cus));
     else
@@ -1496,6 +1502,11 @@ nnhip_status run_matmul_glu(nnhip_ctx* ctx, const char* fn, const void* rp, cons
         {
             // the gated activation in the deep GEMV's epilogue: no y1 round trip
             NNHIP_LAUNCH(fn, launch_gemv_deep(ctx->stream, p));
+            return NNHIP_OK;
+        }
+        if (gemv_split_ok(p, ctx->num_cus))
+        {
+            NNHIP_LAUNCH(fn, launch_gemv_split(ctx->stream, p, ctx->num_cus));
             return NNHIP_OK;
         }
         const nnhip_status st = run_matmul(ctx, fn, rp, tau, xi, s, rowsum, bias, N, K, M, y1);

@@ -809,3 +809,30 @@ def test_between_gemv_and_gemm_gated_and_digits(ctx, orc, N, K, M):
                                torch.nan_to_num(r) if r.is_floating_point() else r)
     finally:
         ctx.set_gemm_tile(0)
+
+
+@pytest.mark.parametrize("N,K,M", [(300, 520, 1), (3000, 3000, 16), (1111, 5000, 7), (4100, 11008, 9), (33, 300, 16)])
+def test_decode_sizes_off_the_deep_gemv(ctx, orc, N, K, M):
+    """Up to 16 tokens on reductions the deep GEMV is not built for: outputs, bias and residual, and the
+    gated activation, bit for bit the oracle's."""
+    import torch
+    say(f"decode size off the deep GEMV N={N} K={K} M={M}")
+    F = N // 2
+    W, X = normal((2 * F, K), N + K, 0.0, 0.02), normal((K, M), N + M)
+    tau = np.abs(W.astype(np.float64)).mean(axis=1).astype(np.float32)
+    b, res = normal((2 * F,), M), normal((2 * F, M), 3 + M)
+    wq = orc.trit_pack(W, tau)
+    dv = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    wd, td = dv(wq.view(np.int32)), dv(tau)
+    rp = ctx.repack(wd, K)
+    acts = ctx.act_quant_i8(dv(X))
+    s = orc.act_scale(X)
+    ref = orc.matmul_q_i8(wq, tau, orc.quantize_i8(X, s, True), s, K, M)
+    assert np.array_equal(ctx.ternary_matmul(rp, td, *acts, 2 * F, K, M).cpu().numpy(), ref)
+    ref = orc.add_row_broadcast(ref.copy(), b)
+    got = ctx.ternary_matmul_add(rp, td, *acts, 2 * F, K, M, dv(res), bias=dv(b))
+    assert np.array_equal(got.cpu().numpy(), ref + res)
+    wo, to, bo = ctx.glu_interleave(wd, td, dv(b), F, K)
+    for act in (0, 1):
+        h = ctx.ternary_matmul_glu(ctx.repack(wo, K), to, *acts, F, K, M, act, bias=bo)
+        assert np.array_equal(h.cpu().numpy(), orc.glu(ref, act))
