@@ -187,34 +187,49 @@ __global__ __launch_bounds__(256) void k_sum_parts(const float* __restrict__ par
 // ---------------------------------------------------------------- matmul_q_t
 
 // Bit transpose of a packed container: A (K, ceil(M/16)) -> At (M, ceil(K/16)), trit (m, k) of
-// At = trit (k, m) of A; codes for k >= K are 2 (trit 0). A block moves a tile of 64 stored
-// rows x 64 words (1024 m): coalesced loads into LDS, then each output word (one m, 16 rows)
-// is gathered from LDS and the 4 words of an m are stored contiguously.
-constexpr int kTpRows = 64, kTpWords = 64;
+// At = trit (k, m) of A; codes for k >= K are 2 (trit 0). A block moves a tile of 256 stored rows x 16
+// words (256 m): a thread takes one word of 16 rows, transposes their 16 x 16 codes in registers (four
+// rounds of block swaps), and the output words meet in LDS so that an m's 16 words are stored together.
+// (Gathering each output word from 16 LDS words took 14.5 us for 6912 x 2560, this 8.0.)
+constexpr int kTpTile = 16;  // words per tile side: 16 of 16 rows each
 __global__ __launch_bounds__(256) void k_trit_transpose(const uint32_t* __restrict__ A, int K, int M,
                                                         uint32_t* __restrict__ At)
 {
-    __shared__ uint32_t tile[kTpRows][kTpWords + 1];
+    // rows 17 words apart and 4 more after every 16: both sides free of bank conflicts
+    constexpr int P = kTpTile + 1, P16 = 16 * P + 4;
+    __shared__ uint32_t tile[kTpTile * P16];
     const int wpa = (M + 15) / 16, wpk = (K + 15) / 16;
-    const int k0 = blockIdx.y * kTpRows, c0 = blockIdx.x * kTpWords;
-    for (int e = threadIdx.x; e < kTpRows * kTpWords; e += 256)
-    {
-        const int r = e / kTpWords, c = e % kTpWords;
-        const int k = k0 + r, col = c0 + c;
-        tile[r][c] = (k < K && col < wpa) ? A[(size_t)k * wpa + col] : 0xAAAAAAAAu;
-    }
-    __syncthreads();
-    // output words: m = 16 * c0 + mm (1024 values), kw = k0 / 16 + q (4 values)
-    for (int e = threadIdx.x; e < 16 * kTpWords * (kTpRows / 16); e += 256)
-    {
-        const int q = e % (kTpRows / 16), mm = e / (kTpRows / 16);
-        const int m = 16 * c0 + mm, kw = k0 / 16 + q;
-        if (m >= M || kw >= wpk) continue;
-        const int c = mm / 16, sh = 2 * (mm % 16);
-        uint32_t word = 0;
+    const int c = threadIdx.x % kTpTile, q = threadIdx.x / kTpTile;
+    const int col = blockIdx.x * kTpTile + c, k0 = (blockIdx.y * kTpTile + q) * 16;
+    uint32_t w[16];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) word |= ((tile[16 * q + i][c] >> sh) & 3u) << (2 * i);
-        At[(size_t)m * wpk + kw] = word;
+    for (int i = 0; i < 16; ++i)
+    {
+        const uint32_t x = A[(size_t)min(k0 + i, K - 1) * wpa + min(col, wpa - 1)];
+        w[i] = k0 + i < K ? x : 0xAAAAAAAAu;
+    }
+    // code j of word i <-> code i of word j: blocks of s x s codes off the diagonal change places
+    constexpr uint32_t kMask[4] = {0x33333333u, 0x0F0F0F0Fu, 0x00FF00FFu, 0x0000FFFFu};
+#pragma unroll
+    for (int b = 3; b >= 0; --b)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+        {
+            const int s = 1 << b;
+            if (i & s) continue;
+            const uint32_t t = ((w[i] >> (2 * s)) ^ w[i + s]) & kMask[b];
+            w[i + s] ^= t;
+            w[i] ^= t << (2 * s);
+        }
+#pragma unroll
+    for (int j = 0; j < 16; ++j) tile[P16 * c + P * j + q] = w[j];
+    __syncthreads();
+    const int kw = blockIdx.y * kTpTile + c;
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+    {
+        const int m = (blockIdx.x * kTpTile + i) * 16 + q;
+        if (m < M && kw < wpk) At[(size_t)m * wpk + kw] = tile[P16 * i + P * q + c];
     }
 }
 
@@ -294,7 +309,7 @@ hipError_t launch_matmul_q(hipStream_t st, const uint32_t* wq, const float* tau,
 hipError_t launch_trit_transpose(hipStream_t st, const uint32_t* A, size_t K, size_t M, uint32_t* At)
 {
     if (K == 0 || M == 0) return hipSuccess;
-    const dim3 tgrid((unsigned)ceil_div(ceil_div(M, 16), (size_t)kTpWords), (unsigned)ceil_div(K, (size_t)kTpRows));
+    const dim3 tgrid((unsigned)ceil_div(M, (size_t)(16 * kTpTile)), (unsigned)ceil_div(K, (size_t)(16 * kTpTile)));
     hipLaunchKernelGGL(k_trit_transpose, tgrid, dim3(256), 0, st, A, (int)K, (int)M, At);
     return hipGetLastError();
 }
@@ -305,7 +320,7 @@ hipError_t launch_matmul_q_t(hipStream_t st, const uint32_t* A, const float* tau
     if (N == 0 || M == 0) return hipSuccess;
     uint32_t* At = reinterpret_cast<uint32_t*>(scratch);
     float* part = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(scratch) + plan.at_bytes);
-    const dim3 tgrid((unsigned)ceil_div(ceil_div(M, 16), (size_t)kTpWords), (unsigned)ceil_div(K, (size_t)kTpRows));
+    const dim3 tgrid((unsigned)ceil_div(M, (size_t)(16 * kTpTile)), (unsigned)ceil_div(K, (size_t)(16 * kTpTile)));
     hipLaunchKernelGGL(k_trit_transpose, tgrid, dim3(256), 0, st, A, (int)K, (int)M, At);
     return run_mq(st, At, nullptr, tau, B, b16, M, K, N, Y, y16, plan, part);
 }

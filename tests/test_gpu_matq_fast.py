@@ -170,6 +170,20 @@ def test_trit_transpose_bits(ctx, orc, K, M):
     assert np.all(ct[:, K:] == 2)
 
 
+@pytest.mark.parametrize("N,K", [(256, 256), (257, 255), (255, 257), (16, 1279), (5, 1281), (33, 2561), (513, 64)])
+def test_absmean_and_transpose_edges(ctx, orc, N, K):
+    """Around the transpose's 256 x 256 tile and the absmean's 20 x 64 columns per round: both exact."""
+    say(f"absmean / trit_transpose N={N} K={K}")
+    W = normal((N, K), 7 * N + K, 0.0, 0.02)
+    W[0, K // 2], W[N // 2, 0] = -0.0, 3e38
+    tau = orc.row_absmean(W)
+    assert np.array_equal(ctx.row_absmean(dev(W)).cpu().numpy(), tau)
+    A = orc.trit_pack(W, tau)
+    At = ctx.trit_transpose(dev(A), K).cpu().numpy().view(np.uint32)
+    codes = lambda P: ((P[:, :, None] >> (2 * np.arange(16, dtype=np.uint32))) & 3).reshape(P.shape[0], -1)
+    assert np.array_equal(codes(At)[:, :N], codes(A)[:, :K].T) and np.all(codes(At)[:, N:] == 2)
+
+
 @pytest.mark.parametrize("K,M,N", [(2560, 6912, 16), (6912, 2560, 4), (2560, 2560, 1), (640, 2560, 7),
                                    (520, 100, 3), (17, 65, 65), (1000, 300, 40)])
 def test_matmul_t_f_gaussian(ctx, orc, K, M, N):
