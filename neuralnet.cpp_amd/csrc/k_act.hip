@@ -8,11 +8,15 @@
 // are bit-identical to the unfused reference sequence whichever kernel runs.
 //
 // Kernels by shape:
-//   k_token_regs   M > 64, K up to 512 * 22: 8 tokens per 16-wave block (M <= 8192 and
-//                  K <= 5120, or K <= 7168 without RMSNorm), else 4 per 8-wave block. Each
+//   k_token_regs   M > 64, K up to 512 * 22: 8 tokens per 16-wave block (mostly M > 1024 and
+//                  K <= 7168), else 4 per 8-wave block. Each
 //                  thread loads its rows (16 B = 4 tokens per row) once and keeps them in
 //                  registers through the passes (sum of squares, absmax, quantize), so X is read
-//                  from HBM exactly once. With RMSNorm a thread's rows are the features of its
+//                  from HBM exactly once. Bound by reading X, and by the L2 requests of the short row
+//                  segments: 2560 x 8192 right after X was written 47.6 -> 27.8 us (3.8 TB/s) with two
+//                  blocks to a CU and the codes not written through; rows off the 16-byte grid
+//                  (2560 x 3333) 58.4 -> 17.1 with 16-byte loads at any alignment.
+//                  With RMSNorm a thread's rows are the features of its
 //                  sum-of-squares part; without it each wave of an 8-token block reads one
 //                  contiguous band of rows. Codes leave through a 4x4 byte transpose in lane
 //                  quads as dword stores.
@@ -32,13 +36,6 @@ namespace
 {
 
 constexpr int kBlock = 256;
-// Cache-policy operand of the register quantizer's xi stores. The 8-token blocks (M <= 8192: a
-// grid of one or a few resident rounds) write the codes through the L2 (kPolicySys) as they are
-// produced: at M = 2048, K = 4096 12.1 -> 10.9 us, RMSNorm 2560 9.35 -> 9.0 us, K = 6912 21.1 ->
-// 20.9 us. The 4-token blocks (larger M, many rounds) keep the default policy, 1-2 % faster
-// there (2560 x 32768: 157.6-159.2 against 160.4-161.0 us).
-template <int TPB>
-constexpr int kXiPolicy = TPB >= 8 ? kPolicySys : 0;
 #ifndef NNHIP_ONE_TOK_MAX_M
 #define NNHIP_ONE_TOK_MAX_M 64  // largest M for k_token_one (K=6912, M=64: 6.8 us per call, the
                                 // 4-token kernel 11.0; equal at K=2560)
@@ -85,16 +82,6 @@ __device__ __forceinline__ float lane_xor(float v)
 // Butterfly over lane bits below 2*OFF (offsets OFF, OFF/2, ..., 1), four values at a time so
 // the lane exchanges of one level overlap. Sum: fl(own + partner), the fixed order of the
 // oracle's tree; max ignores NaN as `a > b ? a : b` does; integer sum is exact.
-template <int OFF>
-__device__ __forceinline__ void bfly_fsum(float (&v)[4])
-{
-    float o[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = lane_xor<OFF>(v[i]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = __fadd_rn(v[i], o[i]);
-    if constexpr (OFF > 1) bfly_fsum<OFF / 2>(v);
-}
 // Max over the same lanes of values that are never NaN and never negative (absolute values,
 // +0 included): their bit patterns order as unsigned integers, so one integer max per level
 // replaces a float compare and select.
@@ -358,11 +345,16 @@ __global__ __launch_bounds__(kTW * kWave) void k_token_lanes(
 template <int TPB>
 constexpr int reg_waves = 2 * TPB;
 
+// Words between the tokens' rows of parts: the lane groups of one store (token quads) fall in
+// different banks.
+template <int TPB>
+constexpr int kRedPitch = kParts + (TPB == 8 ? 8 : 0);
+
 // Everything a block needs to load and finish token groups (uniform across the block).
 template <int TPB>
 struct TokShared
 {
-    float red[kParts][TPB];  // sum-of-squares parts
+    float red[TPB][kRedPitch<TPB>];  // sum-of-squares parts
     float wred[reg_waves<TPB>][TPB];
     int wsum[reg_waves<TPB>][TPB];
     float tok_ri[TPB];
@@ -383,47 +375,55 @@ __device__ __forceinline__ int row_base(int ro)
 template <int R, int TPB, bool kContig>
 constexpr int row_step = kContig ? kWave / (TPB / 4) : reg_waves<TPB> * (kWave / (TPB / 4));
 
-// Issue the loads of group g into x (vector path: one buffer resource over X, K*M*4 < 2^31
-// checked at launch, so rows past K and tokens past M read 0 without a branch).
-template <int R, bool kVec, int TPB, bool kContig = false>
+// Four tokens of a row: 16 bytes at any 4-byte alignment (M may be odd).
+typedef float row4 __attribute__((ext_vector_type(4), aligned(4)));
+
+// Issue the loads of group g into x: one buffer resource over X (K*M*4 < 2^31 checked at launch), so
+// rows past K read 0 without a branch. Threads whose four tokens reach past M read the row's last
+// four and shift (M > 64 here); tokens past M are 0.
+template <int R, int TPB, bool kContig = false>
 __device__ __forceinline__ void load_group(float (&x)[R][4], const TokArgs& a, int g, int ro, int h)
 {
-    const int mt = g * TPB + 4 * h;
+    const int mt = g * TPB + 4 * h, ml = min(mt, a.M - 4);
     const int base = row_base<R, TPB, kContig>(ro);
     constexpr int step = row_step<R, TPB, kContig>;
-    if (kVec)
-    {
-        typedef float v4f __attribute__((ext_vector_type(4)));
-        const __amdgpu_buffer_rsrc_t rx =
-            __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.X), (short)0, a.K * a.M * 4, 0x00020000);
-        const uint32_t moff = mt < a.M ? (uint32_t)mt * 4u : 0x80000000u;
+    const __amdgpu_buffer_rsrc_t rx =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.X), (short)0, a.K * a.M * 4, 0x00020000);
 #pragma unroll
-        for (int r = 0; r < R; ++r)
-        {
-            const v4f v = __builtin_bit_cast(
-                v4f, __builtin_amdgcn_raw_buffer_load_b128(rx, moff + (uint32_t)(base + step * r) * (uint32_t)a.M * 4u, 0, 0));
-            x[r][0] = v[0];
-            x[r][1] = v[1];
-            x[r][2] = v[2];
-            x[r][3] = v[3];
-        }
+    for (int r = 0; r < R; ++r)
+    {
+        const row4 v = __builtin_bit_cast(
+            row4, __builtin_amdgcn_raw_buffer_load_b128(rx, (uint32_t)ml * 4u + (uint32_t)(base + step * r) * (uint32_t)a.M * 4u, 0, 0));
+        x[r][0] = v[0];
+        x[r][1] = v[1];
+        x[r][2] = v[2];
+        x[r][3] = v[3];
     }
-    else
+    if (g * TPB + TPB <= a.M) return;
+    const int d = mt - ml;
+#pragma unroll
+    for (int r = 0; r < R; ++r)
     {
-#pragma unroll
-        for (int r = 0; r < R; ++r)
+        if (d & 1)
         {
-            const int f = base + step * r;
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                x[r][i] = (f < a.K && mt + i < a.M) ? a.X[(size_t)f * a.M + mt + i] : 0.0f;
+            x[r][0] = x[r][1];
+            x[r][1] = x[r][2];
+            x[r][2] = x[r][3];
+            x[r][3] = 0.0f;
         }
+        if (d & 2)
+        {
+            x[r][0] = x[r][2];
+            x[r][1] = x[r][3];
+            x[r][2] = x[r][3] = 0.0f;
+        }
+        if (d >= 4) x[r][0] = x[r][1] = x[r][2] = x[r][3] = 0.0f;
     }
 }
 
 // The three passes over one group held in registers: sum of squares -> rms_inv (RMSNorm),
 // per-token absmax -> scale, quantize -> xi / s / rowsum (and the reference container).
-template <int R, bool kVec, int TPB, bool kNormOK, bool kContig = false>
+template <int R, int TPB, bool kNormOK, bool kContig, int kPolicy>
 __device__ __forceinline__ void finish_group(float (&x)[R][4], const float (&gm)[R], const TokArgs& a,
                                              TokShared<TPB>& sh, int g, int w, int fl, int h, int ro)
 {
@@ -450,23 +450,16 @@ __device__ __forceinline__ void finish_group(float (&x)[R][4], const float (&gm)
 #pragma unroll
         for (int q = 0; q < NP; ++q)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) sh.red[ro + RR * q][4 * h + i] = acc[q][i];
+            for (int i = 0; i < 4; ++i) sh.red[4 * h + i][ro + RR * q] = acc[q][i];
         __syncthreads();
-        if (w == 0)
+        // one wave per token: lane l takes parts l + 64 k (levels 256, 128, 64), then the butterfly
+        if (w < TPB)
         {
-            float sum[4];
+            float v[kParts / kWave];
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-            {
-                float v[kParts / RPW];
-#pragma unroll
-                for (int k = 0; k < kParts / RPW; ++k) v[k] = sh.red[fl + RPW * k][4 * h + i];
-                sum[i] = tree_levels(v);
-            }
-            bfly_fsum<RPW / 2>(sum);
-            if (fl == 0)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) sh.tok_ri[4 * h + i] = rms_inv_of(sum[i], a.inv_f, a.eps);
+            for (int k = 0; k < kParts / kWave; ++k) v[k] = sh.red[w][(threadIdx.x & 63) + kWave * k];
+            const float sum = wave_bfly(tree_levels(v), TqAdd{});
+            if ((threadIdx.x & 63) == 0) sh.tok_ri[w] = rms_inv_of(sum, a.inv_f, a.eps);
         }
         __syncthreads();
         float ri[4];
@@ -487,11 +480,8 @@ __device__ __forceinline__ void finish_group(float (&x)[R][4], const float (&gm)
         {
             const int f = base + step * r;
             if (f >= a.K) continue;
-            if (kVec)
-            {
-                if (mt < a.M)
-                    *reinterpret_cast<float4*>(a.fout + (size_t)f * a.M + mt) = make_float4(x[r][0], x[r][1], x[r][2], x[r][3]);
-            }
+            if (mt + 4 <= a.M)
+                *reinterpret_cast<row4*>(a.fout + (size_t)f * a.M + mt) = row4{x[r][0], x[r][1], x[r][2], x[r][3]};
             else
             {
 #pragma unroll
@@ -605,12 +595,12 @@ __device__ __forceinline__ void finish_group(float (&x)[R][4], const float (&gm)
         {
             // a band's rounds end at Kp in any round (rows past Kp read 0 and are never stored)
             const uint32_t o = q0 + step * r < a.Kp ? xoff + (uint32_t)(step * r) : 0x80000000u;
-            __builtin_amdgcn_raw_buffer_store_b32(col, rxi, o, 0, kXiPolicy<TPB>);
+            __builtin_amdgcn_raw_buffer_store_b32(col, rxi, o, 0, kPolicy);
         }
         else if (r < whole)
-            __builtin_amdgcn_raw_buffer_store_b32(col, rxi, xoff + (uint32_t)(RR * r), 0, kXiPolicy<TPB>);
+            __builtin_amdgcn_raw_buffer_store_b32(col, rxi, xoff + (uint32_t)(RR * r), 0, kPolicy);
         else if (r == whole)
-            __builtin_amdgcn_raw_buffer_store_b32(col, rxi, xpart + (uint32_t)(RR * r), 0, kXiPolicy<TPB>);
+            __builtin_amdgcn_raw_buffer_store_b32(col, rxi, xpart + (uint32_t)(RR * r), 0, kPolicy);
     }
     tsum = bfly_isum1<RPW / 2, 4>(tsum);  // over the quads of the wave's slice
     if (fl < 4) sh.wsum[w][4 * h + j] = tsum;
@@ -632,13 +622,13 @@ __device__ __forceinline__ void finish_group(float (&x)[R][4], const float (&gm)
     }
 }
 
-// One block per token group; block b takes group slot(b), XCD-aware when the group count is a
-// multiple of 8, so the blocks of one XCD take consecutive groups and the groups sharing a
-// 128-byte row segment of X meet in one L2.
-// (R = 12 and 14 with 4-token blocks: at least 3 waves per SIMD, 168 registers; left to itself the
-// compiler took 171 for R = 14, i.e. 2 waves per SIMD, too few loads in flight at prefill sizes)
-template <int R, bool kVec, int TPB, bool kNormOK, bool kContig = false>
-__global__ __launch_bounds__(reg_waves<TPB> * kWave, ((R == 12 || R == 14) && TPB == 4) ? 3 : 1) void k_token_regs(TokArgs a, const float* __restrict__ gamma,
+// One block per token group; the blocks of one XCD (b % 8) take consecutive groups, so the groups
+// sharing a 128-byte row segment of X meet in one L2 (6912 x 3000, whose 750 groups took them in launch
+// order before, 100 -> 36 us).
+// (8 tokens, R <= 5 with RMSNorm: 64 registers for two blocks to a CU, 2560 x 8192 32.1 -> 25.9 us;
+// 4 tokens, R = 12 and 14: at least 3 waves per SIMD, 168 registers)
+template <int R, int TPB, bool kNormOK, bool kContig, int kPolicy>
+__global__ __launch_bounds__(reg_waves<TPB> * kWave, (TPB == 8 && kNormOK && R <= 5) ? 8 : ((R == 12 || R == 14) && TPB == 4) ? 3 : 1) void k_token_regs(TokArgs a, const float* __restrict__ gamma,
                                                                   int n_groups)
 {
     constexpr int RPW = kWave / (TPB / 4);
@@ -649,11 +639,11 @@ __global__ __launch_bounds__(reg_waves<TPB> * kWave, ((R == 12 || R == 14) && TP
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int fl = lane % RPW, h = lane / RPW;  // row within the wave's slice, token quad
     const int ro = RPW * w + fl;
-    const int b = blockIdx.x;
-    const int g = n_groups % 8 == 0 ? (b & 7) * (n_groups >> 3) + (b >> 3) : b;
+    const int b = blockIdx.x, xcd = b & 7;
+    const int g = xcd * (n_groups >> 3) + min(xcd, n_groups & 7) + (b >> 3);
 
     float x[R][4];
-    load_group<R, kVec, TPB, kContig>(x, a, g, ro, h);
+    load_group<R, TPB, kContig>(x, a, g, ro, h);
     float gm[R];
     if (kNormOK && a.norm)
     {
@@ -663,7 +653,7 @@ __global__ __launch_bounds__(reg_waves<TPB> * kWave, ((R == 12 || R == 14) && TP
         for (int r = 0; r < R; ++r)
             gm[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rg, (uint32_t)(RR * r + ro) * 4u, 0, 0));
     }
-    finish_group<R, kVec, TPB, kNormOK, kContig>(x, gm, a, sh, g, w, fl, h, ro);
+    finish_group<R, TPB, kNormOK, kContig, kPolicy>(x, gm, a, sh, g, w, fl, h, ro);
 }
 
 // Decode-sized M (up to 64 tokens): one token per block, 512 threads. Thread t owns sum-of-squares
@@ -847,36 +837,22 @@ __global__ __launch_bounds__(kBlock) void k_to_container(const int8_t* __restric
     }
 }
 
-#ifndef NNHIP_TOK8_MAX_ROUNDS
-#define NNHIP_TOK8_MAX_ROUNDS 10  // largest K/512 rounds for the 8-token register kernel
-#endif
 constexpr size_t kSmallM = 32;
 constexpr size_t kOneTokMaxM = NNHIP_ONE_TOK_MAX_M;
 
-template <int TPB, int R, bool kNormOK = true, bool kContig = false>
-void launch_regs_r(bool vec, hipStream_t st, int n_groups, const TokArgs& a, const float* gamma)
-{
-    auto kern = vec ? k_token_regs<R, true, TPB, kNormOK, kContig> : k_token_regs<R, false, TPB, kNormOK, kContig>;
-    hipLaunchKernelGGL(kern, dim3((unsigned)n_groups), dim3(reg_waves<TPB> * kWave), 0, st, a, gamma, n_groups);
-}
-
 // Launch the instantiation with the smallest R >= rounds from the ascending list Rs; false if
 // none is large enough.
-template <int TPB, int... Rs>
-bool launch_regs_pick(int rounds, bool vec, hipStream_t st, int n_groups, const TokArgs& a, const float* gamma)
+template <int TPB, bool kNormOK, bool kContig, int kPolicy, int... Rs>
+bool launch_regs_pick(int rounds, hipStream_t st, const TokArgs& a, const float* gamma)
 {
+    const int n_groups = (a.M + TPB - 1) / TPB;
+    auto go = [&]<int R>() {
+        hipLaunchKernelGGL((k_token_regs<R, TPB, kNormOK, kContig, kPolicy>), dim3((unsigned)n_groups),
+                           dim3(reg_waves<TPB> * kWave), 0, st, a, gamma, n_groups);
+        return true;
+    };
     bool done = false;
-    ((done = done || (Rs >= rounds && (launch_regs_r<TPB, Rs>(vec, st, n_groups, a, gamma), true))), ...);
-    return done;
-}
-
-// the same without the RMSNorm passes, rows in contiguous bands per wave
-template <int TPB, int... Rs>
-bool launch_regs_pick_contig(int rounds, bool vec, hipStream_t st, int n_groups, const TokArgs& a)
-{
-    bool done = false;
-    ((done = done || (Rs >= rounds && (launch_regs_r<TPB, Rs, false, true>(vec, st, n_groups, a, nullptr), true))),
-     ...);
+    ((done = done || (Rs >= rounds && go.template operator()<Rs>())), ...);
     return done;
 }
 
@@ -903,29 +879,33 @@ static hipError_t launch_token_kernel(hipStream_t st, const float* X, const floa
     }
     if (rounds <= 22 && (K + 4096) * M * 4 < 0x7FFFFFFFull)
     {
-        // rows are read as float4 when every row start is 16-byte aligned
-        const bool vec = M % 4 == 0 && reinterpret_cast<uintptr_t>(X) % 16 == 0 &&
-                         (fout == nullptr || reinterpret_cast<uintptr_t>(fout) % 16 == 0);
-        // 8 tokens per block (32-byte row segments, 16 waves) while a thread's rows fit the
-        // 128 registers of a 1024-thread block and the grid is at most a few rounds (K=4096,
-        // M=2048: 14.2 against 15.7 us; 2560 x 32768, where the smaller blocks keep more waves
-        // resident: 193 against 159 us); 4 tokens (16-byte segments, 8 waves) otherwise
+        // 8 tokens per block (32-byte row segments: half the L2 requests of 16-byte ones) where 4-token
+        // blocks would be more than one to a CU (M > 1024; below, the smaller blocks use more CUs: X
+        // just written, K = 2560, M = 512 9.4 against 11.0 us, K = 6912, M = 1024 17.4 against 20.2)
+        // and a thread's rows fit the 128 registers of a 1024-thread block (K <= 7168). Measured the
+        // same way, 8 against 4 tokens: 2560 x 8192 27.8 / 34.5 us, 2560 x 32768 138 / 169, 4096 x 8192
+        // 48 / 59, 6912 x 8192 90 / 96; with RMSNorm past 10 rounds 6912 x 4096 43.8 / 42.4 and
+        // 6912 x 3333 (rows off the 16-byte grid) 40.0 / 45.4, so those take 8 from M = 4096 or M % 4.
         TokArgs a{X, norm, eps, inv_f, (int)K, (int)M, (int)Kp, mode, xi, s, rowsum, xq_ref, fout};
-        // Without RMSNorm the 8-token layout also serves 11 to 14 rounds (K <= 7168: the FFN
-        // width 6912): those instantiations leave the norm passes out, which keeps them within
-        // the 128 registers (K=6912, M=2048: 16-byte segments read the 56 MB at ~4 TB/s).
-        const bool tok8 = vec && M <= 8192 && (rounds <= NNHIP_TOK8_MAX_ROUNDS || (!norm && mode == 0 && rounds <= 14));
-        const int n_groups = (int)ceil_div(M, (size_t)(tok8 ? 8 : 4));
+        const bool plain = !norm && mode == 0;
+        const bool tok8 = M > 1024 && rounds <= 14 && (plain || rounds <= 10 || M > 4096 || M % 4 != 0);
+        // One resident round of 8-token blocks (M <= 2048) writes the codes through the L2 as they are
+        // produced: 4096 x 2048 13.9 -> 12.6 us. More rounds don't: right after X was written it cost
+        // 4096 x 8192 48 -> 69 us, 6912 x 8192 86 -> 129.
+        const bool thru = M <= 2048 && rounds <= 10;
         // Without RMSNorm (mode 0) the 8-token blocks read each wave's rows as one contiguous band
         // (the absmax and the code sums do not depend on the order): K=4096, M=2048 11.1 -> 10.3 us,
         // K=6912 21.6-22.1 -> 19.8-20.1 us, the same codes (A/B of two builds on one box).
         bool launched;
-        if (tok8 && !norm && mode == 0)
-            launched = launch_regs_pick_contig<8, 1, 2, 3, 4, 5, 6, 8, 10, 12, 14>(rounds, vec, st, n_groups, a);
+        if (tok8 && plain)
+            launched = thru ? launch_regs_pick<8, false, true, kPolicySys, 1, 2, 3, 4, 5, 6, 8, 10>(rounds, st, a, gamma)
+                            : launch_regs_pick<8, false, true, 0, 1, 2, 3, 4, 5, 6, 8, 10, 12, 14>(rounds, st, a, gamma);
+        else if (tok8)
+            launched = thru ? launch_regs_pick<8, true, false, kPolicySys, 1, 2, 3, 4, 5, 6, 8, 10>(rounds, st, a, gamma)
+                            : launch_regs_pick<8, true, false, 0, 1, 2, 3, 4, 5, 6, 8, 10, 12, 14>(rounds, st, a, gamma);
         else
-            launched = tok8 ? launch_regs_pick<8, 1, 2, 3, 4, 5, 6, 8, 10>(rounds, vec, st, n_groups, a, gamma)
-                            : launch_regs_pick<4, 1, 2, 3, 4, 5, 6, 8, 10, 12, 14, 16, 18, 20, 22>(rounds, vec, st,
-                                                                                                n_groups, a, gamma);
+            launched = launch_regs_pick<4, true, false, 0, 1, 2, 3, 4, 5, 6, 8, 10, 12, 14, 16, 18, 20, 22>(rounds, st, a,
+                                                                                                      gamma);
         if (launched) return hipGetLastError();
     }
     if (M <= kSmallM)

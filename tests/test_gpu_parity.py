@@ -209,6 +209,35 @@ def test_rmsnorm_quant(ctx, orc, F, M, eps):
     assert np.array_equal(host(xi)[:, :F], orc.container_to_int8(xq_o, M).T)
 
 
+@pytest.mark.parametrize("F,M", [(40, 65), (600, 1027), (2560, 1033), (2561, 2049), (4096, 2051), (640, 4102), (6912, 67),
+                                 (6912, 1029), (6913, 4100), (7169, 1026), (11000, 71)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_token_blocks_edges(ctx, orc, F, M, shift):
+    """Both block sizes at ragged token counts, M % 4 of every kind and X off its 16-byte grid: the
+    codes, scales and sums with and without RMSNorm, the container and RMSNorm alone, all exact."""
+    say(f"token blocks F={F} M={M} shift={shift}")
+    X = normal((F, M), F + M, 0.0, 1.0)
+    X[F // 2, M - 1], X[0, 0] = 30.0, -40.0
+    import torch
+    buf = torch.empty(F * M + shift, device="cuda")
+    Xd = buf[shift:].view(F, M)
+    Xd.copy_(dev(X))
+    g = normal((F,), 3, 1.0, 0.1)
+    for norm in (False, True):
+        if norm:
+            xi, s, rs, xq = ctx.rmsnorm_quant_i8(Xd, dev(g), 1e-6, want_container=True)
+            xq_o, s_o = orc.rmsnorm_quant_i8(X, g, 1e-6)
+        else:
+            xi, s, rs, xq = ctx.act_quant_i8(Xd, want_container=True)
+            s_o = orc.act_scale(X)
+            xq_o = orc.quantize_i8(X, s_o, True)
+        q = orc.container_to_int8(xq_o, M).T
+        assert np.array_equal(host(s), s_o) and np.array_equal(host(xq, np.uint32), xq_o)
+        assert np.array_equal(host(xi)[:, :F], q) and np.all(host(xi)[:, F:] == 0)
+        assert np.array_equal(host(rs), q.astype(np.int64).sum(axis=1))
+    assert np.array_equal(host(ctx.rmsnorm(Xd, dev(g), 1e-6)), orc.rmsnorm(X, g, 1e-6))
+
+
 @pytest.mark.parametrize("F,M,loc", [(2560, 33, 0.0), (6912, 64, 3.0), (1, 5, 0.0), (17, 1, -1.0), (300, 1000, 0.5),
                                      (13, 2048, 0.0), (2560, 31, 0.0)])
 def test_layernorm(ctx, orc, F, M, loc):
