@@ -94,8 +94,9 @@ nnhip_status nnhip_ctx_get_stream(nnhip_ctx* ctx, void** stream);
 
 /* Block tile of the prefill GEMM (M > 16 tokens): automatic (the default) picks, per call, the
  * tile with the fewest estimated block rounds over the CUs, and may split the rows over two
- * launches (256 x 128 blocks over whole rounds of the CUs, a smaller tile over the rest); the
- * others force one tile for all rows. A tuning control of this library (the reference's GEMM
+ * launches (256 x 128 blocks over whole rounds of the CUs, a smaller tile over the rest), or take
+ * blocks that split the reduction over their waves where the tiles are few (17 to a few hundred
+ * tokens); the others force one tile for all rows. A tuning control of this library (the reference's GEMM
  * shader has a single 64 x 64 tile); results are bit-identical whichever tile runs. */
 #define NNHIP_GEMM_TILE_AUTO 0
 #define NNHIP_GEMM_TILE_256x128 1
@@ -596,7 +597,7 @@ nnhip_status nnhip_kv_cache_fill_h(nnhip_ctx* ctx, const float* k, const float* 
 /* Causal attention of the T tokens over caches already holding rows [0, pos0 + T) (after
  * nnhip_kv_cache_fill): out (H*dk, B*T), column b*T + t = per query head h the softmax
  * ((rot(q_h) . K^T) * scale) . V over cache rows [0, pos0 + t] of sequence b, KV head h / (H/Hkv),
- * q rotated at pos0 + t. f32 on the fp32 MFMA with an online softmax: within 2e-6 relative of a
+ * q rotated at pos0 + t. f32 operands as two f16 halves on the f16 MFMA with an online softmax: within 2e-6 relative of a
  * float64 evaluation (the reference does not pin the order). dk in {64, 128}; H / Hkv in
  * {1, 2, 4, 8}. Replaces the attention steps of T AttentionBase::forward_step calls
  * (compute_layer_attention.hpp:1022-1083). */

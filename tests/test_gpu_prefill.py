@@ -6,7 +6,7 @@ compute_layer_attention.hpp:1003-1091), then the whole prefill of Decoder.prefil
 
 The cache rows (rotated keys, values) are compared bit for bit. The attention output is compared
 within 5e-6 x max(1, max|out|) of the oracle: its dot products and softmax sums are f32 in an
-order the reference leaves open, and the prefill kernel accumulates on the fp32 MFMA with an
+order the reference leaves open, and the prefill kernel sums f16-half products in f32 with an
 online softmax.
 """
 import math
