@@ -842,7 +842,7 @@ hipError_t launch_embed(hipStream_t st, const float* table, const int32_t* ids, 
 {
     // below a tile of tokens the scattered stores are few (48 tokens 3.0 against 3.3 us, 64 3.3 both,
     // 128 4.4 against 3.4)
-    if (!tm && B >= kEmbTile)
+    if (!tm && B >= kEmbTile && ceil_div(d, kEmbTile) <= 65535)  // (grid limit)
     {
         k_embed_cols<<<dim3((unsigned)ceil_div(B, kEmbTile), (unsigned)ceil_div(d, kEmbTile)), kSmallBlock, 0, st>>>(
             table, ids, (int)V, (int)d, (int)B, out);

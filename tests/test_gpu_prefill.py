@@ -448,3 +448,13 @@ def test_embedding_gather_many_tokens(ctx, V, d, B):
     ref = table[np.clip(ids, 0, V - 1)].T.copy()
     ref[:, [3, B - 1]] = np.nan
     assert same_bits(host(ctx.embedding_gather(dev(table), dev(ids))), ref)
+
+
+def test_embedding_gather_more_features_than_tiles(ctx):
+    """More 64-feature tiles than a grid's second dimension takes: one element per thread instead."""
+    import torch
+    d, B = 64 * 65535 + 1, 64
+    table = torch.arange(2 * d, device="cuda", dtype=torch.float32).reshape(2, d)
+    ids = (torch.arange(B, device="cuda") % 2).to(torch.int32)
+    out = ctx.embedding_gather(table, ids)
+    assert all(torch.equal(out[:, b], table[b % 2]) for b in range(B))
