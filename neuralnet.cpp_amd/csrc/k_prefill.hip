@@ -25,8 +25,8 @@
 // are. Sums, softmax and output are f32, and sums of 16 products at a time round less often than
 // the fp32 MFMA's pairs: against float64, 4 x 2048 tokens of 20 heads over 5 KV heads of 128 are
 // 4.6e-7 off (f32 products: 6.7e-7), 3 x 1111 at position 517 6.7e-7 (9.7e-7).
-// What the halves cannot hold (infinities, NaN, a tile's largest value outside 2^+-48) sends the
-// work-group to the f32 products (attend_f32).
+// What the halves cannot hold (infinities, NaN, a tile's largest value outside 2^+-48, scores that
+// may pass 2^20) sends the work-group to the f32 products (attend_f32).
 //
 // Work-group = 8 waves = (the R = H / Hkv heads of KV head g) x (8 / R blocks of 32 queries) of
 // sequence b; all waves share each 32-key tile of K and V, staged in LDS as f16 planes (double
@@ -187,6 +187,9 @@ constexpr int kPThreads = 64 * kPWaves;
 constexpr int kPExpMax = 48;           // scalings beyond 2^+-48 take the f32 products
 constexpr float kPLazy = 8.0f;         // log2 growth of a query's maximum before its sums are rescaled
 constexpr float kPBias = 6.0f;         // probabilities are held times 2^6: at most 2^14 with the growth
+// Largest score in log2 units. The rounding of a query's reference maximum is then at most 2^-4; with
+// larger scores it alone would take probabilities out of f16's range.
+constexpr float kPReach = 0x1p20f;
 
 struct PrefillArgs
 {
@@ -234,8 +237,8 @@ __device__ __forceinline__ void split2(float x0, float x1, v2h& hi, v2h& lo)
 __device__ __forceinline__ float pow2(int e) { return __builtin_bit_cast(float, (uint32_t)(127 + e) << 23); }
 
 // The exponent that brings values whose largest bit pattern is mx (sign cleared) into [2^14, 2^15):
-// 0 for all-zero values. Outside +-kPExpMax (infinities and NaN among it) the f32 products run.
-__device__ __forceinline__ int f16_exp(uint32_t mx) { return mx == 0 ? 0 : 14 + 127 - (int)(mx >> 23); }
+// kPExpMax for all-zero values. Outside +-kPExpMax (infinities and NaN among it) the f32 products run.
+__device__ __forceinline__ int f16_exp(uint32_t mx) { return mx == 0 ? kPExpMax : 14 + 127 - (int)(mx >> 23); }
 
 // The wave's largest value
 __device__ __forceinline__ uint32_t wave_max(uint32_t v)
@@ -309,7 +312,8 @@ __device__ __forceinline__ void store_out(const PrefillArgs& a, const PrefillWav
 }
 
 // The work-group's attention on the fp32 MFMA (v_mfma_f32_32x32x2_f32), for inputs that the f16
-// halves cannot hold: infinities, NaN, or a tile whose largest value is outside 2^+-48. Per 32-key
+// halves cannot hold: infinities, NaN, a tile whose largest value is outside 2^+-48, or scores that may
+// pass 2^20. Per 32-key
 // tile S^T (not S) is in the accumulators, so lane l holds query l % 32 and keys
 // 8(v/4) + 4(l/32) + v%4 of its 16 elements v: the B operand of the P . V products when the keys of
 // product s are taken in that order. The sum over the head dimension takes product s = 4c + e over
@@ -515,6 +519,7 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
         }
     };
     int ek = 0, ev = 1 << 20;  // exponents of the staged tile: K's own, V's running smallest
+    float eqf = 0.0f;          // the lane's query: 2^-eq |scale| log2(e)
     // the tile's exponents, then raw as f16 halves into buffer kb & 1
     auto convert = [&](int kb, int* flag) {
         uint8_t* buf = smem + (kb & 1) * Tile::kBuf;
@@ -530,6 +535,8 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
                 if (tid == 0) *flag = 1;
                 ek = ev = 0;
             }
+            // products of halves are below 2^30, DK of them to a score
+            else if (__builtin_amdgcn_ballot_w64(eqf * pow2(-ek) > kPReach / (DK * 0x1p30f)) != 0 && lane == 0) *flag = 1;
         }
         const float sv = F32C ? pow2(ev > kPExpMax ? 0 : ev) : 1.0f, sk = F32C ? pow2(ek) : 1.0f;
         if (is_v)
@@ -621,7 +628,6 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
 
     // ---- the lane's rotated query in halves: step c holds dimensions 16c + 8h + 0..7, scaled by 2^eq
     v8h qh[NC], ql[NC];
-    float eqf = 0.0f;  // 2^-eq |scale| log2(e)
     if (w.live)
     {
         float qv[DK / 2];
@@ -654,6 +660,7 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
 #pragma unroll
     for (int d = 0; d < ND; ++d) o[d] = v16f{};
     float m_ref = -__builtin_inff(), l_run = 0.0f;  // log2 units; l_run: this lane half's keys
+    float m_abs = 0.0f;                             // f16 caches, whose scale is not looked up: largest |m_ref|
     int eo = 0;                                     // the exponent of V in o
 
     post_max(0);
@@ -736,6 +743,7 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
 #pragma unroll
                     for (int v = 0; v < 16; ++v) o[d][v] *= corr;
                 m_ref = m_new;
+                if constexpr (!F32C) m_abs = fmaxf(m_abs, fabsf(m_new));
             }
             const float mb = kPBias - m_ref;
             v8h ph[2], pl[2];
@@ -776,7 +784,7 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
     if constexpr (!F32C)
     {
         // f16 caches are not looked through for infinities and NaN: any that matters is in the sums
-        bool bad = !(fabsf(l_run) < __builtin_inff());
+        bool bad = !(fabsf(l_run) < __builtin_inff()) || m_abs > kPReach;
 #pragma unroll
         for (int d = 0; d < ND; ++d)
 #pragma unroll

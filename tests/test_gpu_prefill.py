@@ -405,6 +405,27 @@ def test_prefill_halves_match_float64(ctx, H, Hkv, dk, T, pos0, f16):
 
 
 @pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("H,Hkv,dk,T,pos0", [(4, 1, 128, 200, 0), (2, 2, 64, 70, 90)])
+def test_prefill_large_scores(ctx, H, Hkv, dk, T, pos0, f16):
+    """Finite queries and keys whose scores pass 2^20, in every tile or in one that comes late: a query's
+    weight is on its best key (the next is thousands lower, an f32 score's rounding a few units), so the
+    output is that key's value row, here against float64."""
+    B, max_len = 2, pos0 + T
+    scale = float(np.float32(1.0 / np.sqrt(dk)))
+    cdt = np.float16 if f16 else np.float32
+    for aq, ak, late in [(1e4, 1e4, 1.0), (3e5, 3e3, 1.0)] + ([] if f16 else [(1e6, 1e6, 1.0), (1.0, 1.0, 2.0 ** 30)]):
+        say(f"prefill large scores H={H} Hkv={Hkv} dk={dk} T={T} f16={f16} q x {aq} k x {ak} late x {late}")
+        q = normal((H * dk, B * T), 960) * np.float32(aq)
+        kc = normal((B, max_len, Hkv * dk), 961) * np.float32(ak)
+        kc[:, max_len - T // 3] *= np.float32(late)
+        kc, vc = kc.astype(cdt), normal((B, max_len, Hkv * dk), 962).astype(cdt)
+        got = host(ctx.attention_prefill(dev(q), dev(kc), dev(vc), B, T, H, Hkv, dk, pos0, scale)).astype(np.float64)
+        ref, mag = attend64(q, kc, vc, B, T, H, Hkv, dk, pos0, scale)
+        err = np.abs(got - ref) / mag
+        assert float(err.max()) <= 1e-5, float(err.max())
+
+
+@pytest.mark.parametrize("f16", [False, True])
 def test_prefill_special_values(ctx, f16):
     """A NaN or infinite key makes exactly the queries that see it NaN (+inf scores: inf - inf), a NaN
     query its own head's column; a zero or negative scale and all-zero values are ordinary. The other
