@@ -16,20 +16,23 @@
 // Hkv*dk) as the decode step's; cos / sin (max_len, dk/2).
 //
 // k_attn_prefill: the fp32 MFMA's rate (157 TFLOP/s) bounded this attention (101 of it at 4 x 2048
-// tokens), and the f16 MFMA runs 16 times as fast. So the products run on v_mfma_f32_32x32x16_f16
-// with every f32 operand as the sum of two f16 halves, x 2^e = hi + lo: e brings the operand's
-// largest value (of a query; of a tile of K; of V so far) to 2^14..2^15, hi and lo are rounded to
-// nearest, so the pair holds x to 2^-24 of itself (to 2^-39 of the largest value for elements far
-// below it). Products of halves are exact in f32; low x low (below 2^-24 of a term) is left out:
-// three MFMAs per product with f32 caches, two with f16 caches, whose elements are halves as they
-// are. Sums, softmax and output are f32, and sums of 16 products at a time round less often than
-// the fp32 MFMA's pairs: against float64, 4 x 2048 tokens of 20 heads over 5 KV heads of 128 are
-// 4.6e-7 off (f32 products: 6.7e-7), 3 x 1111 at position 517 6.7e-7 (9.7e-7).
-// What the halves cannot hold (infinities, NaN, a tile's largest value outside 2^+-48, scores that
-// may pass 2^20) sends the work-group to the f32 products (attend_f32).
+// tokens), and the f16 and bf16 MFMAs run 16 times as fast. So its products run on those with every
+// f32 operand as a sum of parts, whose products are exact in f32:
+//   * S = K . Q^T: two f16 halves, x 2^e = hi + lo to 2^-23 of x, where e brings the largest value of a
+//     query or of a tile of K to 2^14..2^15 (f16 caches: K as it is). low x low, at most 2^-22 of a
+//     term, is left out: three MFMAs per product with f32 caches, two with f16 caches.
+//   * O = P . V: three bf16 parts, x = b0 + b1 + b2 exactly and without a scale, two for f16 caches' V.
+//     The probability of a key and the size of its value have nothing to do with each other, so
+//     neither may cost the other bits: no exponent shared by a tile or a sequence holds both (f16
+//     halves of V under one scale lost a channel 1e-7 of the others to 1e-4, 1e-10 altogether).
+//     Products b_i b_j with i + j > 2, at most 2^-24 of a term, are left out: six and five MFMAs.
+// Sums, softmax and output are f32. Against float64, 1024 tokens of 20 heads over 5 KV heads of 128,
+// f32 / f16 caches: 2.3e-7 / 2.0e-7 off in norm (f32 products: 3.9e-7 both).
+// What the parts cannot hold (infinities, NaN, a query's or K tile's largest value outside 2^+-48,
+// outputs below 2^-100, scores that may pass 2^20) sends the work-group to the f32 products (attend_f32).
 //
 // Work-group = 8 waves = (the R = H / Hkv heads of KV head g) x (8 / R blocks of 32 queries) of
-// sequence b; all waves share each 32-key tile of K and V, staged in LDS as f16 planes (double
+// sequence b; all waves share each 32-key tile of K and V, staged in LDS as planes of parts (double
 // buffered, one barrier per tile): the next tile is converted from registers while the one after
 // it is loaded. A wave computes S^T = K . Q^T (32 keys x 32 queries) and O^T += V^T . P^T, where
 // lane l holds query l % 32 throughout: its 16 elements v of S^T are keys 8(v/4) + 4(l/32) + v%4,
@@ -37,11 +40,12 @@
 // V^T is dimension (DK/32) r + d, which lets a staging lane load contiguous dimensions and its
 // stores fall on all banks. K rows and V^T rows are padded to odd multiples of 16 bytes.
 // Softmax in log2 units with the hardware exp2; a query's reference maximum moves only when it has
-// grown by 2^8 (probabilities are held times 2^6, at most 2^14), so the sums are rarely rescaled.
+// grown by 2^8 (probabilities are at most 2^8), so the sums are rarely rescaled.
 // Work-groups are issued heaviest first (the last query blocks attend over the most keys).
-// Measured (calls back to back, us, f32 products / here): f32 caches 4 x 2048 tokens 848 / 328,
-// 3 x 1111 at 517 432 / 162, 16 x 2048 3077 / 1119, 1 x 64 21.9 / 13.9; f16 caches 821 / 209,
-// 426 / 105, 3132 / 774, 22.0 / 12.8.
+// Measured (calls back to back in a graph, us, f32 products / here): f32 caches 4 x 2048 tokens
+// 809 / 398, 3 x 1111 at 517 411 / 202, 16 x 2048 3088 / 1498, 1 x 64 22.5 / 17.7; f16 caches 817 / 293,
+// 421 / 146, 3153 / 1121, 22.7 / 15.9. Two f16 halves for P and V too (at the cost above) took 295 and
+// 198 us at 4 x 2048.
 // Caches of f16 elements (compute = F16): the fill rounds the rotated keys and the values to the
 // nearest f16 (ties to even), as the decode append does.
 #include "common.hpp"
@@ -181,15 +185,16 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef float v2f __attribute__((ext_vector_type(2)));
+typedef __bf16 v8b __attribute__((ext_vector_type(8)));
+typedef __bf16 v2b __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kPWaves = 8;             // waves of a work-group: R heads x (8 / R) blocks of 32 queries
 constexpr int kPThreads = 64 * kPWaves;
 constexpr int kPExpMax = 48;           // scalings beyond 2^+-48 take the f32 products
 constexpr float kPLazy = 8.0f;         // log2 growth of a query's maximum before its sums are rescaled
-constexpr float kPBias = 6.0f;         // probabilities are held times 2^6: at most 2^14 with the growth
-// Largest score in log2 units. The rounding of a query's reference maximum is then at most 2^-4; with
-// larger scores it alone would take probabilities out of f16's range.
-constexpr float kPReach = 0x1p20f;
+constexpr float kPReach = 0x1p20f;     // largest score in log2 units: the reference maximum rounds by 2^-4
+constexpr float kPTiny = 0x1p-100f;    // outputs below this (but for 0) may have lost bits of a bf16 part
 
 struct PrefillArgs
 {
@@ -208,20 +213,21 @@ struct PrefillArgs
 template <int DK, typename CT>
 struct PrefillTile
 {
-    static constexpr int kPlanes = sizeof(CT) == 4 ? 2 : 1;  // high and low f16 halves of f32 values
+    static constexpr int kKPlanes = sizeof(CT) == 4 ? 2 : 1;  // K: high and low f16 halves of f32 values
+    static constexpr int kVPlanes = sizeof(CT) == 4 ? 3 : 2;  // V: bf16 parts of f32 / f16 values
     // rows are padded by 16 bytes: 16 lanes' reads of consecutive rows fall on all banks, and every
     // chunk is at a constant offset from a lane's first
     static constexpr int kKPitch = DK * 2 + 16, kVPitch = kPK * 2 + 16;
     static constexpr int kKPlane = kPK * kKPitch, kVPlane = DK * kVPitch;
-    static constexpr int kV = kPlanes * kKPlane;             // K planes, then V planes
-    static constexpr int kBuf = kV + kPlanes * kVPlane;
+    static constexpr int kV = kKPlanes * kKPlane;            // K planes, then V planes
+    static constexpr int kBuf = kV + kVPlanes * kVPlane;
     static constexpr int KROW = DK + 4;                      // f32 products: padded row (floats)
     static constexpr int kF32 = 2 * kPK * KROW * 4;
     static constexpr int kMain = 2 * kBuf > kF32 ? 2 * kBuf : kF32;  // double-buffered
-    static constexpr int kBytes = kMain + 128;               // maxima of two tiles, the fallback flag
+    static constexpr int kBytes = kMain + 64;                // maxima of K in two tiles, the fallback flag
 };
 
-// The two halves of four f32 values scaled into f16's range: x = hi + lo up to 2^-24 |x| or 2^-25
+// The two halves of two f32 values scaled into f16's range: x = hi + lo up to 2^-23 |x| or 2^-25
 __device__ __forceinline__ void split2(float x0, float x1, v2h& hi, v2h& lo)
 {
     hi = __builtin_convertvector(v2f{x0, x1}, v2h);
@@ -231,6 +237,22 @@ __device__ __forceinline__ void split2(float x0, float x1, v2h& hi, v2h& lo)
     asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(l0) : "v"(u), "v"(x0));
     asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(l1) : "v"(u), "v"(x1));
     lo = __builtin_convertvector(v2f{l0, l1}, v2h);
+}
+
+// The first N bf16 parts of two values: x = sum of parts, exactly, for f32 values (N = 3) and widened f16
+// values (N = 2) from 2^-110 on (each rounding leaves 8 bits less); infinities and NaN give NaN.
+template <int N>
+__device__ __forceinline__ void split_bf16(float x0, float x1, v2b (&part)[N])
+{
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+    {
+        part[n] = __builtin_convertvector(v2f{x0, x1}, v2b);
+        if (n + 1 == N) break;
+        const uint32_t u = __builtin_bit_cast(uint32_t, part[n]);
+        x0 -= __builtin_bit_cast(float, u << 16);
+        x1 -= __builtin_bit_cast(float, u & 0xFFFF0000u);
+    }
 }
 
 // 2^e for |e| <= 126
@@ -312,8 +334,7 @@ __device__ __forceinline__ void store_out(const PrefillArgs& a, const PrefillWav
 }
 
 // The work-group's attention on the fp32 MFMA (v_mfma_f32_32x32x2_f32), for inputs that the f16
-// halves cannot hold: infinities, NaN, a tile whose largest value is outside 2^+-48, or scores that may
-// pass 2^20. Per 32-key
+// and bf16 parts cannot hold (see the top of the file). Per 32-key
 // tile S^T (not S) is in the accumulators, so lane l holds query l % 32 and keys
 // 8(v/4) + 4(l/32) + v%4 of its 16 elements v: the B operand of the P . V products when the keys of
 // product s are taken in that order. The sum over the head dimension takes product s = 4c + e over
@@ -412,10 +433,10 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
     constexpr int CH = DK / 8;   // 16-byte chunks of a K row
     constexpr int KU = CH * kPK / 256;  // chunks a thread stages
     extern __shared__ __align__(16) uint8_t smem[];
-    uint32_t* smax = reinterpret_cast<uint32_t*>(smem + Tile::kMain);  // [2][8]: per tile parity and wave
+    uint32_t* smax = reinterpret_cast<uint32_t*>(smem + Tile::kMain);  // [2][4]: per tile parity and K wave
     // set to send the work-group to the f32 products: written in iteration kb (or before the loop) into
     // [(kb + 1) & 1] and read after the barrier of iteration kb + 1, so all waves read the same value
-    int* sflag = reinterpret_cast<int*>(smem + Tile::kMain + 64);
+    int* sflag = reinterpret_cast<int*>(smem + Tile::kMain + 32);
 
     const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, l32 = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -483,7 +504,6 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
                 }
                 else if constexpr (W == 2)
                 {
-                    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
                     const u32x2 x = __builtin_amdgcn_raw_buffer_load_b64(rt, at[i], 0, 0);
                     raw[2 * i] = x[0];
                     raw[2 * i + 1] = x[1];
@@ -507,38 +527,33 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
     // words of raw in use
     constexpr int VW = 4 * ND * (int)sizeof(CT) / 4, KW = KU * 8 * (int)sizeof(CT) / 4;
     static_assert(VW == KW && VW <= RW, "V and K threads stage the same amount");
-    // f32 caches: the wave's largest magnitude, for the tile's scaling
+    // f32 caches: the wave's largest magnitude in K, for the tile's scaling
     auto post_max = [&](int kb) {
-        if constexpr (F32C)
-        {
-            uint32_t mx = 0;
+        if (!F32C || is_v) return;
+        uint32_t mx = 0;
 #pragma unroll
-            for (int e = 0; e < VW; ++e) mx = max(mx, raw[e] & 0x7FFFFFFFu);
-            mx = wave_max(mx);
-            if (lane == 0) smax[(kb & 1) * 8 + wave] = mx;
-        }
+        for (int e = 0; e < KW; ++e) mx = max(mx, raw[e] & 0x7FFFFFFFu);
+        mx = wave_max(mx);
+        if (lane == 0) smax[(kb & 1) * 4 + wave - 4] = mx;
     };
-    int ek = 0, ev = 1 << 20;  // exponents of the staged tile: K's own, V's running smallest
-    float eqf = 0.0f;          // the lane's query: 2^-eq |scale| log2(e)
-    // the tile's exponents, then raw as f16 halves into buffer kb & 1
+    int ek = 0;        // exponent of the staged tile's K
+    float eqf = 0.0f;  // the lane's query: 2^-eq |scale| log2(e)
+    // K's exponent, then raw as f16 halves (K) and bf16 parts (V) into buffer kb & 1
     auto convert = [&](int kb, int* flag) {
         uint8_t* buf = smem + (kb & 1) * Tile::kBuf;
         if constexpr (F32C)
         {
-            const uint32_t* sm = smax + (kb & 1) * 8;
-            const uint32_t mv = max(max(sm[0], sm[1]), max(sm[2], sm[3])), mk = max(max(sm[4], sm[5]), max(sm[6], sm[7]));
-            ek = __builtin_amdgcn_readfirstlane(f16_exp(mk));
-            const int e = __builtin_amdgcn_readfirstlane(f16_exp(mv));
-            if (mv != 0) ev = min(ev, e);
-            if (abs(ek) > kPExpMax || abs(e) > kPExpMax)
+            const uint32_t* sm = smax + (kb & 1) * 4;
+            ek = __builtin_amdgcn_readfirstlane(f16_exp(max(max(sm[0], sm[1]), max(sm[2], sm[3]))));
+            if (abs(ek) > kPExpMax)
             {
                 if (tid == 0) *flag = 1;
-                ek = ev = 0;
+                ek = 0;
             }
-            // products of halves are below 2^30, DK of them to a score
+            // products of halves are at most 2^30, DK of them to a score
             else if (__builtin_amdgcn_ballot_w64(eqf * pow2(-ek) > kPReach / (DK * 0x1p30f)) != 0 && lane == 0) *flag = 1;
         }
-        const float sv = F32C ? pow2(ev > kPExpMax ? 0 : ev) : 1.0f, sk = F32C ? pow2(ek) : 1.0f;
+        const float sk = F32C ? pow2(ek) : 1.0f;
         if (is_v)
         {
             // row 32e + vg = dimension ND vg + e; its 4 chunks are (16-key half s, lane half) and hold
@@ -549,26 +564,20 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
             {
                 const int r = 32 * e + vg;
                 uint8_t* dst = buf + Tile::kV + r * Tile::kVPitch + 32 * s + 16 * hh + 8 * ah;
-                if constexpr (F32C)
-                {
-                    float x[4];
+                float x[4];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) x[i] = __builtin_bit_cast(float, raw[ND * i + e]) * sv;
-                    v2h h0, h1, l0, l1;
-                    split2(x[0], x[1], h0, l0);
-                    split2(x[2], x[3], h1, l1);
-                    *reinterpret_cast<v4h*>(dst) = v4h{h0[0], h0[1], h1[0], h1[1]};
-                    *reinterpret_cast<v4h*>(dst + Tile::kVPlane) = v4h{l0[0], l0[1], l1[0], l1[1]};
-                }
-                else
+                for (int i = 0; i < 4; ++i)
                 {
-                    // half e of each key's words
-                    constexpr int W = ND / 2;
-                    const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
-                    uint32_t* d = reinterpret_cast<uint32_t*>(dst);
-                    d[0] = __builtin_amdgcn_perm(raw[W + e / 2], raw[e / 2], sel);
-                    d[1] = __builtin_amdgcn_perm(raw[3 * W + e / 2], raw[2 * W + e / 2], sel);
+                    if constexpr (F32C) x[i] = __builtin_bit_cast(float, raw[ND * i + e]);
+                    else x[i] = (float)__builtin_bit_cast(v2h, raw[ND / 2 * i + e / 2])[e & 1];
                 }
+                v2b p0[Tile::kVPlanes], p1[Tile::kVPlanes];
+                split_bf16(x[0], x[1], p0);
+                split_bf16(x[2], x[3], p1);
+#pragma unroll
+                for (int q = 0; q < Tile::kVPlanes; ++q)
+                    *reinterpret_cast<u32x2*>(dst + q * Tile::kVPlane) =
+                        u32x2{__builtin_bit_cast(uint32_t, p0[q]), __builtin_bit_cast(uint32_t, p1[q])};
             }
         }
         else
@@ -598,29 +607,29 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
         }
     };
 
-    // Fragments from LDS, four 16-byte reads at a time, a group ahead of the products that use them:
-    // group g of K holds steps GS g .., group g of V^T (block, half) pairs GS g .., each with its low
-    // plane next to it for f32 caches.
-    constexpr int GS = 4 / Tile::kPlanes;
-    static_assert(NC % GS == 0 && (2 * ND) % GS == 0, "whole groups");
+    // Fragments from LDS, up to four 16-byte reads at a time, a group ahead of the products that use them:
+    // group g of K holds steps GK g .., group g of V^T (block, half) pairs GV g .., each with its planes.
+    constexpr int PK = Tile::kKPlanes, PV = Tile::kVPlanes, GK = 4 / PK, GV = 4 / PV;
+    constexpr int GKN = NC / GK, GVN = 2 * ND / GV;  // groups
+    static_assert(NC % GK == 0 && (2 * ND) % GV == 0, "whole groups");
     const uint32_t k_at = (uint32_t)(l32 * Tile::kKPitch + 16 * h), v_at = (uint32_t)(Tile::kV + l32 * Tile::kVPitch + 16 * h);
-    auto read_k = [&](v8h(&f)[4], uint32_t par, int g) {
+    auto read_k = [&](u32x4(&f)[4], uint32_t par, int g) {
         const uint8_t* p = smem + (par + k_at);
 #pragma unroll
-        for (int e = 0; e < GS; ++e)
+        for (int e = 0; e < GK; ++e)
 #pragma unroll
-            for (int q = 0; q < Tile::kPlanes; ++q)
-                f[Tile::kPlanes * e + q] = *reinterpret_cast<const v8h*>(p + 32 * (GS * g + e) + q * Tile::kKPlane);
+            for (int q = 0; q < PK; ++q)
+                f[PK * e + q] = *reinterpret_cast<const u32x4*>(p + 32 * (GK * g + e) + q * Tile::kKPlane);
     };
-    auto read_v = [&](v8h(&f)[4], uint32_t par, int g) {
+    auto read_v = [&](u32x4(&f)[4], uint32_t par, int g) {
         const uint8_t* p = smem + (par + v_at);
 #pragma unroll
-        for (int e = 0; e < GS; ++e)
+        for (int e = 0; e < GV; ++e)
         {
-            const int d = (GS * g + e) >> 1, t = (GS * g + e) & 1;
+            const int d = (GV * g + e) >> 1, t = (GV * g + e) & 1;
 #pragma unroll
-            for (int q = 0; q < Tile::kPlanes; ++q)
-                f[Tile::kPlanes * e + q] = *reinterpret_cast<const v8h*>(p + 32 * d * Tile::kVPitch + 32 * t + q * Tile::kVPlane);
+            for (int q = 0; q < PV; ++q)
+                f[PV * e + q] = *reinterpret_cast<const u32x4*>(p + 32 * d * Tile::kVPitch + 32 * t + q * Tile::kVPlane);
         }
     };
 
@@ -661,7 +670,6 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
     for (int d = 0; d < ND; ++d) o[d] = v16f{};
     float m_ref = -__builtin_inff(), l_run = 0.0f;  // log2 units; l_run: this lane half's keys
     float m_abs = 0.0f;                             // f16 caches, whose scale is not looked up: largest |m_ref|
-    int eo = 0;                                     // the exponent of V in o
 
     post_max(0);
     __syncthreads();
@@ -680,10 +688,10 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
             fallback = true;
             break;
         }
-        const int ek_now = ek, ev_now = ev;
+        const int ek_now = ek;
         // this tile's first K fragments, in flight during the conversion of the next tile
         const uint32_t par = (uint32_t)(kb & 1) * Tile::kBuf;
-        v8h fr[2][4];
+        u32x4 fr[2][4];
         read_k(fr[0], par, 0);
         __builtin_amdgcn_sched_barrier(0);
         if (kb + 1 < nkb)
@@ -696,17 +704,18 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
             // S^T = K . Q^T: the products of the halves but low x low (2^-24 of a term)
             v16f s = v16f{};
 #pragma unroll
-            for (int g = 0; g < NC / GS; ++g)
+            for (int g = 0; g < GKN; ++g)
             {
-                if (g + 1 < NC / GS) read_k(fr[(g + 1) & 1], par, g + 1);
+                if (g + 1 < GKN) read_k(fr[(g + 1) & 1], par, g + 1);
                 else read_v(fr[(g + 1) & 1], par, 0);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int e = 0; e < GS; ++e)
+                for (int e = 0; e < GK; ++e)
                 {
-                    const int c = GS * g + e;
-                    const v8h kh = fr[g & 1][Tile::kPlanes * e];
-                    if constexpr (F32C) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[g & 1][2 * e + 1], qh[c], s, 0, 0, 0);
+                    const int c = GK * g + e;
+                    const v8h kh = __builtin_bit_cast(v8h, fr[g & 1][PK * e]);
+                    if constexpr (F32C)
+                        s = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, fr[g & 1][PK * e + 1]), qh[c], s, 0, 0, 0);
                     s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, ql[c], s, 0, 0, 0);
                     s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, qh[c], s, 0, 0, 0);
                 }
@@ -727,17 +736,11 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
             mx = fmaxf(mx, __shfl_xor(mx, 32)) * f;
             // the reference of a query moves only when its maximum has grown by 2^8 (or is new)
             const bool grown = mx > m_ref + kPLazy;
-            if (__builtin_amdgcn_ballot_w64(grown) != 0 || (F32C && ev_now != eo))
+            if (__builtin_amdgcn_ballot_w64(grown) != 0)
             {
                 const float m_new = grown ? mx : m_ref;
-                float corr = __builtin_amdgcn_exp2f(m_ref - m_new);  // 0 on the first tile
+                const float corr = __builtin_amdgcn_exp2f(m_ref - m_new);  // 0 on the first tile
                 l_run *= corr;
-                if (F32C && ev_now != eo)
-                {
-                    // V's exponent went down (the first tile: nothing summed yet)
-                    if (kb > 0) corr *= pow2(max(ev_now - eo, -126));
-                    eo = ev_now;
-                }
 #pragma unroll
                 for (int d = 0; d < ND; ++d)
 #pragma unroll
@@ -745,65 +748,71 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
                 m_ref = m_new;
                 if constexpr (!F32C) m_abs = fmaxf(m_abs, fabsf(m_new));
             }
-            const float mb = kPBias - m_ref;
-            v8h ph[2], pl[2];
+            v8b p[3][2];
 #pragma unroll
             for (int v = 0; v < 16; v += 2)
             {
-                const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[v], f, mb));
-                const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[v + 1], f, mb));
+                const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[v], f, -m_ref));
+                const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[v + 1], f, -m_ref));
                 l_run += p0;
                 l_run += p1;
-                v2h x, y;
-                split2(p0, p1, x, y);
-                ph[v >> 3][v & 7] = x[0], ph[v >> 3][(v & 7) + 1] = x[1];
-                pl[v >> 3][v & 7] = y[0], pl[v >> 3][(v & 7) + 1] = y[1];
+                v2b x[3];
+                split_bf16(p0, p1, x);
+#pragma unroll
+                for (int q = 0; q < 3; ++q) p[q][v >> 3][v & 7] = x[q][0], p[q][v >> 3][(v & 7) + 1] = x[q][1];
             }
             __builtin_amdgcn_sched_barrier(0);
-            // O^T += V^T . P^T
+            // O^T += V^T . P^T: the products of parts i and j with i + j <= 2, smallest first; the rest is
+            // at most 2^-24 of a term. A tile is summed from zero and added once: that rounds the running
+            // sum once in 32 keys. The add of a block runs beside the products of the next.
+            v16f sum[2];
 #pragma unroll
-            for (int g = 0; g < 2 * ND / GS; ++g)
+            for (int g = 0; g < GVN; ++g)
             {
-                const v8h(&f4)[4] = fr[(NC / GS + g) & 1];
-                if (g + 1 < 2 * ND / GS) read_v(fr[(NC / GS + g + 1) & 1], par, g + 1);
+                const u32x4(&f4)[4] = fr[(GKN + g) & 1];
+                if (g + 1 < GVN) read_v(fr[(GKN + g + 1) & 1], par, g + 1);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int e = 0; e < GS; ++e)
+                for (int e = 0; e < GV; ++e)
                 {
-                    const int d = (GS * g + e) >> 1, t = (GS * g + e) & 1;
-                    const v8h vh = f4[Tile::kPlanes * e];
-                    if constexpr (F32C) o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f4[2 * e + 1], ph[t], o[d], 0, 0, 0);
-                    o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, pl[t], o[d], 0, 0, 0);
-                    o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, ph[t], o[d], 0, 0, 0);
+                    const int d = (GV * g + e) >> 1, t = (GV * g + e) & 1;
+                    if (t == 0) sum[d & 1] = v16f{};
+                    if (t == 1 - (GV & 1) && d > 0) o[d - 1] += sum[(d - 1) & 1];
+#pragma unroll
+                    for (int n = 2; n >= 0; --n)
+#pragma unroll
+                        for (int i = PV - 1 < n ? PV - 1 : n; i >= 0; --i)
+                            sum[d & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8b, f4[PV * e + i]), p[n - i][t], sum[d & 1], 0, 0, 0);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
+            o[ND - 1] += sum[(ND - 1) & 1];
         }
         if (kb + 2 < nkb) post_max(kb + 2);
     }
-    if constexpr (!F32C)
-    {
-        // f16 caches are not looked through for infinities and NaN: any that matters is in the sums
-        bool bad = !(fabsf(l_run) < __builtin_inff()) || m_abs > kPReach;
+    // V is not looked through for infinities and NaN, nor f16 caches' K: any that matters is in the sums.
+    // Nor for values whose smallest part would lie below bf16's range: their output is tiny then.
+    l_run += __shfl_xor(l_run, 32);
+    bool bad = !(l_run < __builtin_inff()) || m_abs > kPReach;
 #pragma unroll
-        for (int d = 0; d < ND; ++d)
+    for (int d = 0; d < ND; ++d)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) bad |= !(fabsf(o[d][v]) < __builtin_inff());
-        fallback = __syncthreads_or(!fallback && w.live && bad) || fallback;
-    }
-    if (fallback)
+        for (int v = 0; v < 16; ++v)
+        {
+            const float y = fabsf(o[d][v]);
+            bad |= !(y < __builtin_inff()) || (y < l_run * kPTiny && y != 0.0f);
+        }
+    if (__syncthreads_or(!fallback && w.live && bad) || fallback)
     {
         attend_f32<DK, CT>(a, w, last_key, rk, rv, reinterpret_cast<float*>(smem));
         return;
     }
-    l_run += __shfl_xor(l_run, 32);
     if (!w.live) return;
-    // o / l (correctly rounded but for the last step's double rounding: the residual is exact) and
-    // V's exponent back; an all-zero V has none
-    const float r = 1.0f / l_run, back = F32C ? pow2(eo > kPExpMax ? 0 : -eo) : 1.0f;
+    // o / l, correctly rounded but for the last step's double rounding: the residual is exact
+    const float r = 1.0f / l_run;
     store_out<DK>(a, w, h, [](int d, int i) { return ND * i + d; }, [&](int d, int v) {
-        const float q = o[d][v] * r, y = __builtin_fmaf(__builtin_fmaf(-q, l_run, o[d][v]), r, q);
-        return F32C ? y * back : y;
+        const float q = o[d][v] * r;
+        return __builtin_fmaf(__builtin_fmaf(-q, l_run, o[d][v]), r, q);
     });
 }
 

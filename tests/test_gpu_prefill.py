@@ -405,6 +405,41 @@ def test_prefill_halves_match_float64(ctx, H, Hkv, dk, T, pos0, f16):
 
 
 @pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("H,Hkv,dk,T,pos0", [(4, 1, 128, 300, 5), (4, 4, 64, 150, 90)])
+def test_prefill_value_spread(ctx, H, Hkv, dk, T, pos0, f16):
+    """Each output is as exact as its own sum |p v|, whatever other values its tile holds: channels far
+    below the others, one value row far above them (earlier with next to no weight, and masked for the
+    queries before it), all values tiny. Within 5e-6 of sum |p v|: exponents of magnitude up to 12 round
+    by 12 x 2^-24 in a score and again in the product with log2(e), sums of 305 keys by about 2e-6."""
+    B, max_len = 1, pos0 + T
+    scale = float(np.float32(1.0 / np.sqrt(dk)))
+    q, kc, vc = normal((H * dk, B * T), 970), normal((B, max_len, Hkv * dk), 971), normal((B, max_len, Hkv * dk), 972)
+
+    def check(label, q, k, v):
+        say(f"prefill value spread H={H} Hkv={Hkv} dk={dk} T={T} f16={f16} {label}")
+        k, v = (a.astype(np.float16 if f16 else np.float32) for a in (k, v))
+        got = host(ctx.attention_prefill(dev(q), dev(k), dev(v), B, T, H, Hkv, dk, pos0, scale)).astype(np.float64)
+        ref, mag = attend64(q, k, v, B, T, H, Hkv, dk, pos0, scale)
+        err = np.where(mag > 0, np.abs(got - ref) / np.where(mag > 0, mag, 1.0), got != 0)
+        assert float(err.max()) <= 5e-6, (label, float(err.max()))
+
+    for e in (1e-4,) if f16 else (1e-7, 1e-10, 1e-20, 1e-35):
+        v = vc.copy()
+        v[..., 5::dk] *= np.float32(e)
+        check(f"channel x {e}", q, kc, v)
+    for e in (8, 14) if f16 else (8, 14, 25, 33):
+        v, k = vc * np.float32(2.0 ** -e if f16 else 1.0), kc.copy()
+        late, early = v.copy(), v.copy()
+        late[:, max_len - T // 2] *= np.float32(2.0 ** e)
+        check(f"row 2^{e} in the middle", q, k, late)
+        early[:, 3] *= np.float32(2.0 ** e)
+        k[:, 3] = -3.0
+        check(f"row 2^{e} early, next to no weight", np.abs(q), k, early)
+    for e in (1e-3, 1e-5) if f16 else (1e-20, 1e-30, 1e-36):
+        check(f"all values x {e}", q, kc, vc * np.float32(e))
+
+
+@pytest.mark.parametrize("f16", [False, True])
 @pytest.mark.parametrize("H,Hkv,dk,T,pos0", [(4, 1, 128, 200, 0), (2, 2, 64, 70, 90)])
 def test_prefill_large_scores(ctx, H, Hkv, dk, T, pos0, f16):
     """Finite queries and keys whose scores pass 2^20, in every tile or in one that comes late: a query's
