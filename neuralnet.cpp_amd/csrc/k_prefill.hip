@@ -19,8 +19,9 @@
 // tokens), and the f16 and bf16 MFMAs run 16 times as fast. So its products run on those with every
 // f32 operand as a sum of parts, whose products are exact in f32:
 //   * S = K . Q^T: two f16 halves, x 2^e = hi + lo to 2^-23 of x, where e brings the largest value of a
-//     query or of a tile of K to 2^14..2^15 (f16 caches: K as it is). low x low, at most 2^-22 of a
-//     term, is left out: three MFMAs per product with f32 caches, two with f16 caches.
+//     query or of a tile of K to 2^14..2^15 (f16 caches: K as it is). What is below 2^-40 of that is
+//     lost, less than 2^-21 of a score in all where scores cannot reach 2^18. low x low, at most
+//     2^-22 of a term, is left out: three MFMAs per product with f32 caches, two with f16 caches.
 //   * O = P . V: three bf16 parts, x = b0 + b1 + b2 exactly and without a scale, two for f16 caches' V.
 //     The probability of a key and the size of its value have nothing to do with each other, so
 //     neither may cost the other bits: no exponent shared by a tile or a sequence holds both (f16
@@ -29,7 +30,8 @@
 // Sums, softmax and output are f32. Against float64, 1024 tokens of 20 heads over 5 KV heads of 128,
 // f32 / f16 caches: 2.3e-7 / 2.0e-7 off in norm (f32 products: 3.9e-7 both).
 // What the parts cannot hold (infinities, NaN, a query's or K tile's largest value outside 2^+-48,
-// outputs below 2^-100, scores that may pass 2^20) sends the work-group to the f32 products (attend_f32).
+// outputs below 2^-100, largest values whose scores could reach 2^18) sends the work-group to the f32
+// products (attend_f32).
 //
 // Work-group = 8 waves = (the R = H / Hkv heads of KV head g) x (8 / R blocks of 32 queries) of
 // sequence b; all waves share each 32-key tile of K and V, staged in LDS as planes of parts (double
@@ -188,12 +190,15 @@ typedef float v2f __attribute__((ext_vector_type(2)));
 typedef __bf16 v8b __attribute__((ext_vector_type(8)));
 typedef __bf16 v2b __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kPWaves = 8;             // waves of a work-group: R heads x (8 / R) blocks of 32 queries
 constexpr int kPThreads = 64 * kPWaves;
 constexpr int kPExpMax = 48;           // scalings beyond 2^+-48 take the f32 products
 constexpr float kPLazy = 8.0f;         // log2 growth of a query's maximum before its sums are rescaled
-constexpr float kPReach = 0x1p20f;     // largest score in log2 units: the reference maximum rounds by 2^-4
+// Largest dk max|q| max|k| |scale| log2(e) of a query and a tile: a score's parts below the halves' range
+// (2^-40 of the largest value) add up to less than 2^-21, and no score rounds a reference maximum by 2^-5.
+constexpr float kPReach = 0x1p18f;
 constexpr float kPTiny = 0x1p-100f;    // outputs below this (but for 0) may have lost bits of a bf16 part
 
 struct PrefillArgs
@@ -433,7 +438,7 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
     constexpr int CH = DK / 8;   // 16-byte chunks of a K row
     constexpr int KU = CH * kPK / 256;  // chunks a thread stages
     extern __shared__ __align__(16) uint8_t smem[];
-    uint32_t* smax = reinterpret_cast<uint32_t*>(smem + Tile::kMain);  // [2][4]: per tile parity and K wave
+    uint32_t* smax = reinterpret_cast<uint32_t*>(smem + Tile::kMain);  // [2][4]: per tile parity and K wave; f16 caches: [8] per wave
     // set to send the work-group to the f32 products: written in iteration kb (or before the loop) into
     // [(kb + 1) & 1] and read after the barrier of iteration kb + 1, so all waves read the same value
     int* sflag = reinterpret_cast<int*>(smem + Tile::kMain + 32);
@@ -538,6 +543,7 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
     };
     int ek = 0;        // exponent of the staged tile's K
     float eqf = 0.0f;  // the lane's query: 2^-eq |scale| log2(e)
+    float klim = 0.0f; // f16 caches: the largest key element within kPReach of every query of the work-group
     // K's exponent, then raw as f16 halves (K) and bf16 parts (V) into buffer kb & 1
     auto convert = [&](int kb, int* flag) {
         uint8_t* buf = smem + (kb & 1) * Tile::kBuf;
@@ -550,8 +556,16 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
                 if (tid == 0) *flag = 1;
                 ek = 0;
             }
-            // products of halves are at most 2^30, DK of them to a score
+            // |q| 2^eq and |k| 2^ek are at most 2^15
             else if (__builtin_amdgcn_ballot_w64(eqf * pow2(-ek) > kPReach / (DK * 0x1p30f)) != 0 && lane == 0) *flag = 1;
+        }
+        else if (!is_v)
+        {
+            u16x2 m = {0, 0};
+#pragma unroll
+            for (int e = 0; e < KW; ++e) m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2, raw[e] & 0x7FFF7FFFu));
+            const uint16_t top = max(m[0], m[1]);
+            if (__builtin_amdgcn_ballot_w64(!((float)__builtin_bit_cast(_Float16, top) <= klim)) != 0 && lane == 0) *flag = 1;
         }
         const float sk = F32C ? pow2(ek) : 1.0f;
         if (is_v)
@@ -669,10 +683,21 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
 #pragma unroll
     for (int d = 0; d < ND; ++d) o[d] = v16f{};
     float m_ref = -__builtin_inff(), l_run = 0.0f;  // log2 units; l_run: this lane half's keys
-    float m_abs = 0.0f;                             // f16 caches, whose scale is not looked up: largest |m_ref|
 
     post_max(0);
+    if constexpr (!F32C)
+    {
+        const uint32_t mx = wave_max(__builtin_bit_cast(uint32_t, eqf));  // not negative
+        if (lane == 0) smax[wave] = mx;
+    }
     __syncthreads();
+    if constexpr (!F32C)
+    {
+        uint32_t mx = 0;
+#pragma unroll
+        for (int i = 0; i < kPWaves; ++i) mx = max(mx, smax[i]);
+        klim = kPReach / (DK * 0x1p15f) / __builtin_bit_cast(float, mx);  // |q| 2^eq is at most 2^15
+    }
     convert(0, sflag);
     if (nkb > 1)
     {
@@ -746,7 +771,6 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
 #pragma unroll
                     for (int v = 0; v < 16; ++v) o[d][v] *= corr;
                 m_ref = m_new;
-                if constexpr (!F32C) m_abs = fmaxf(m_abs, fabsf(m_new));
             }
             v8b p[3][2];
 #pragma unroll
@@ -790,10 +814,9 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
         }
         if (kb + 2 < nkb) post_max(kb + 2);
     }
-    // V is not looked through for infinities and NaN, nor f16 caches' K: any that matters is in the sums.
-    // Nor for values whose smallest part would lie below bf16's range: their output is tiny then.
+    // V is not looked through for infinities and NaN: any that matters is in the sums. Nor for values whose smallest part would lie below bf16's range: their output is tiny then.
     l_run += __shfl_xor(l_run, 32);
-    bool bad = !(l_run < __builtin_inff()) || m_abs > kPReach;
+    bool bad = !(l_run < __builtin_inff());
 #pragma unroll
     for (int d = 0; d < ND; ++d)
 #pragma unroll

@@ -440,6 +440,41 @@ def test_prefill_value_spread(ctx, H, Hkv, dk, T, pos0, f16):
 
 
 @pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("H,Hkv,dk,T,pos0", [(4, 1, 128, 300, 5), (4, 4, 64, 150, 90)])
+def test_prefill_score_spread(ctx, H, Hkv, dk, T, pos0, f16):
+    """A score is as exact as its own terms, whatever else its query or its tile of keys holds: a channel
+    far above the others in the queries where the keys are 0, in the keys where the queries are 0, and a
+    key row far above the others that the queries before it don't see. Within 5e-6 of sum |p v| as above
+    (the queries that see the row put their weight on it or none)."""
+    B, max_len = 1, pos0 + T
+    scale = float(np.float32(1.0 / np.sqrt(dk)))
+    q, kc, vc = normal((H * dk, B * T), 980), normal((B, max_len, Hkv * dk), 981), normal((B, max_len, Hkv * dk), 982)
+
+    def check(label, q, k):
+        say(f"prefill score spread H={H} Hkv={Hkv} dk={dk} T={T} f16={f16} {label}")
+        k, v = (a.astype(np.float16 if f16 else np.float32) for a in (k, vc))
+        got = host(ctx.attention_prefill(dev(q), dev(k), dev(v), B, T, H, Hkv, dk, pos0, scale)).astype(np.float64)
+        ref, mag = attend64(q, k, v, B, T, H, Hkv, dk, pos0, scale)
+        err = np.abs(got - ref) / mag
+        assert float(err.max()) <= 5e-6, (label, float(err.max()))
+
+    for e in (8, 16, 24, 32, 45):
+        q2, k2 = q.copy(), kc.copy()
+        q2[5::dk] *= np.float32(2.0 ** e)
+        k2[..., 5::dk] = 0.0
+        check(f"query channel 2^{e}", q2, k2)
+    for e in (8, 13) if f16 else (8, 16, 24, 32, 45):
+        q2, k2 = q.copy(), kc.copy()
+        q2[5::dk] = 0.0
+        k2[..., 5::dk] *= np.float32(2.0 ** e)
+        check(f"key channel 2^{e}", q2, k2)
+    for e in (13,) if f16 else (20, 30):
+        k2 = kc.copy()
+        k2[:, max_len - 3] *= np.float32(2.0 ** e)
+        check(f"key row 2^{e}", q, k2)
+
+
+@pytest.mark.parametrize("f16", [False, True])
 @pytest.mark.parametrize("H,Hkv,dk,T,pos0", [(4, 1, 128, 200, 0), (2, 2, 64, 70, 90)])
 def test_prefill_large_scores(ctx, H, Hkv, dk, T, pos0, f16):
     """Finite queries and keys whose scores pass 2^20, in every tile or in one that comes late: a query's
