@@ -52,6 +52,21 @@ __device__ __forceinline__ int code_at(const uint32_t* rp, int KT, int n, int k)
 // Y[n, m] of a token holding a NaN or an infinity: the finite terms cannot change a NaN or an
 // infinite total, so only the non-finite ones are evaluated (IEEE products tau_n * trit * x):
 // NaN if any is NaN (0 x inf included) or infinities of both signs meet, else that infinity.
+__device__ __forceinline__ void add_special(bool& nan, bool& pos, bool& neg, float tw, float x)
+{
+    if (x != x || tw != tw || tw == 0.0f)
+        nan = true;
+    else if ((tw > 0.0f) == (x > 0.0f))
+        pos = true;
+    else
+        neg = true;
+}
+
+__device__ __forceinline__ float special_total(bool nan, bool pos, bool neg)
+{
+    return (nan || (pos && neg)) ? __builtin_nanf("") : (pos ? __builtin_inff() : -__builtin_inff());
+}
+
 __device__ float special_dot(const void* B, bool b16, const float* kscale, const uint32_t* rp, int KT, int K, int M,
                              int n, int m, float tn)
 {
@@ -60,24 +75,47 @@ __device__ float special_dot(const void* B, bool b16, const float* kscale, const
     {
         const float x = load_bk(B, kscale, k, M, m, b16);
         if (fabsf(x) <= 3.4028234663852886e38f) continue;
-        const float tw = tn * (float)(code_at(rp, KT, n, k) - 2);
-        if (x != x || tw != tw || tw == 0.0f)
-            nan = true;
-        else if ((tw > 0.0f) == (x > 0.0f))
-            pos = true;
-        else
-            neg = true;
+        add_special(nan, pos, neg, tn * (float)(code_at(rp, KT, n, k) - 2), x);
     }
-    return (nan || (pos && neg)) ? __builtin_nanf("") : (pos ? __builtin_inff() : -__builtin_inff());
+    return special_total(nan, pos, neg);
 }
 
-// A special token's outputs for rows n0, n0 + step, ... (the GEMM epilogue leaves them alone)
+// A special token's outputs, by one wave: rows 64 c + lane for chunks c = c0, c0 + step, ... (the GEMM
+// epilogue leaves them alone). A lane reads every 64th element, and the wave stops at the few that are not
+// finite, or once all its rows are NaN: one element after the other per row is a chain of K memory
+// latencies for each row (whole products with one such token: 6912 x 2560, 2048 tokens 31 ms so, 7.5 ms
+// with a thread per output, here 0.18 ms of which 0.16 for finite tokens; 2560 x 6912, 8 tokens 8.4, 0.91
+// and 0.03 ms).
 __device__ void write_specials(const DigitSpecials& sp, const void* B, bool b16, const float* kscale, int K, int Kp, int M,
-                               int m, int n0, int step)
+                               int m, int c0, int step)
 {
-    for (int n = n0; n < sp.N; n += step)
+    constexpr int U = 8;  // loads in flight per lane
+    const int lane = threadIdx.x & 63;
+    for (int c = c0; 64 * c < sp.N; c += step)
     {
-        const float y = special_dot(B, b16, kscale, sp.rp, Kp / kTileK, K, M, n, m, sp.tau ? sp.tau[n] : 1.0f);
+        const int n = min(64 * c + lane, sp.N - 1);
+        const float tn = sp.tau ? sp.tau[n] : 1.0f;
+        bool nan = false, pos = false, neg = false;
+        for (int k0 = 0; k0 < K && __builtin_amdgcn_ballot_w64(!nan) != 0; k0 += 64 * U)
+        {
+            float x[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) x[u] = load_bk(B, kscale, min(k0 + 64 * u + lane, K - 1), M, m, b16);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+            {
+                // (past the end the last element again, which changes nothing)
+                uint64_t at = __builtin_amdgcn_ballot_w64(!(fabsf(x[u]) <= 3.4028234663852886e38f));
+                for (; at != 0 && __builtin_amdgcn_ballot_w64(!nan) != 0; at &= at - 1)
+                {
+                    const int l = __builtin_ctzll(at);
+                    const float y = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x[u]), l));
+                    add_special(nan, pos, neg, tn * (float)(code_at(sp.rp, Kp / kTileK, n, min(k0 + 64 * u + l, K - 1)) - 2), y);
+                }
+            }
+        }
+        if (64 * c + lane >= sp.N) continue;
+        const float y = special_total(nan, pos, neg);
         const size_t o = (size_t)n * M + m;
         if (sp.y16) reinterpret_cast<_Float16*>(sp.y)[o] = (_Float16)y;
         else reinterpret_cast<float*>(sp.y)[o] = y;
@@ -185,7 +223,7 @@ __global__ __launch_bounds__(kDigThreads) void k_digits(const void* __restrict__
         rowsum[4 * m + tid] = t;
     }
     if (tid == 0) ex[m] = bad ? kDigitSpecial : E;
-    if (bad && sp.y) write_specials(sp, B, f16, kscale, K, Kp, M, m, tid, kDigThreads);
+    if (bad && sp.y) write_specials(sp, B, f16, kscale, K, Kp, M, m, tid >> 6, NW);
 }
 
 // The digits of many tokens (M > 4) in two launches that read B along tokens, 64 at a time, so
@@ -321,9 +359,10 @@ __global__ __launch_bounds__(kDigRowThreads) void k_digit_rows(const void* __res
     const int p = w;  // one digit per wave
     if (m < M)
         atomicAdd(&rowsum[4 * m + p], ssum[0][p][lane] + ssum[1][p][lane] + ssum[2][p][lane] + ssum[3][p][lane]);
-    // the rows of a special token, shared out over the blocks of its tokens
-    if (sp.y && m < M && bad)
-        write_specials(sp, B, sizeof(BT) == 2, kscale, K, Kp, M, m, blockIdx.y * NW + w, gridDim.y * NW);
+    // the rows of the special tokens, shared out over the waves of the blocks of these tokens
+    if (!sp.y) return;
+    for (uint64_t todo = __builtin_amdgcn_ballot_w64(m < M && bad); todo != 0; todo &= todo - 1)
+        write_specials(sp, B, sizeof(BT) == 2, kscale, K, Kp, M, m0 + __builtin_ctzll(todo), blockIdx.y * NW + w, gridDim.y * NW);
 }
 
 // The same digits for a few long tokens (the split-k path, M <= 4): block (c, m) takes columns

@@ -419,3 +419,46 @@ def test_matmul_f_many_tokens_bits(ctx, orc, N, K, M, b16):
     trT = orc.trits_of(At.cpu().numpy().view(np.uint32), K)
     assert same_bits(got[:, fin], digit_model(trT, X[:, fin], kscale=tauT))
     check(got[:, bad], orc.matmul_q_t(A, tauT, np.ascontiguousarray(X[:, bad]), N), TOL)
+
+
+@pytest.mark.parametrize("N,K,M", [(70, 515, 6), (300, 4100, 5), (129, 5000, 70), (64, 1, 67), (193, 513, 600)])
+def test_matmul_f_special_tokens(ctx, orc, N, K, M):
+    """Tokens with infinities and NaN among finite ones where the digit kernels write them (M > 4): at the
+    ends of K, several in one row, every token of a group of 64, tails of rows and of the 512 elements a
+    wave looks at. The same NaN and infinities as the reference product's, and f32 of its finite outputs."""
+    say(f"ternary_matmul_f special tokens N={N} K={K} M={M}")
+    wq, tau, rp = case(ctx, orc, N, K, seed=N + K + M)
+    X = normal((K, M), 90 + M)
+    X[0, 0], X[K - 1, 1], X[K // 2, 3] = np.inf, np.nan, -np.inf
+    X[[0, K // 3, K - 1], 4] = np.inf, -np.inf, np.inf
+    X[(np.arange(64, M) * 37) % K, np.arange(64, M)] = np.inf
+    got = host(ctx.ternary_matmul_f(rp, dev(tau), dev(X), N, K))
+    check(got, orc.matmul_q(wq, tau, X, K), TOL)
+
+
+@pytest.mark.parametrize("N,K,M", [(6912, 2560, 512), (2560, 6912, 8), (2560, 2560, 40)])
+def test_matmul_f_special_token_time(ctx, N, K, M):
+    """One token with a NaN takes the product no more than 15 times as long (1.1 to 4 times here; element
+    after element for each row it was 80 to 400 times)."""
+    import torch
+    say(f"ternary_matmul_f special token time N={N} K={K} M={M}")
+    W = torch.randn((N, K), device="cuda") * 0.02
+    tau = ctx.row_absmean(W)
+    rp = ctx.repack(ctx.trit_pack(W, tau), K)
+    X = torch.randn((K, M), device="cuda")
+    X2 = X.clone()
+    X2[K // 2, M // 2] = float("nan")
+
+    def best(x):
+        e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        t = []
+        for _ in range(4):
+            e[0].record()
+            for _ in range(5):
+                ctx.ternary_matmul_f(rp, tau, x, N, K)
+            e[1].record()
+            e[1].synchronize()
+            t.append(e[0].elapsed_time(e[1]))
+        return min(t)
+
+    assert best(X2) <= 15.0 * best(X)
