@@ -44,8 +44,11 @@ __global__ void k_fill_u32(uint32_t* __restrict__ dst, uint32_t value, size_t wo
 
 // One wave per row: lane l sums fl(|w| * fl(1/K)) for k = l, l+64, ... in ascending order,
 // then a xor butterfly over 32,16,8,4,2,1 (commutative pairs, so every lane ends with the
-// same value). Matches orc_row_absmean bit for bit. Bound by HBM: 4NK bytes read; 20 loads in flight
-// per lane (one at a time the 6912 x 2560 matrix took 23-25 us, so 12.4: 5.7 TB/s).
+// same value). Matches orc_row_absmean bit for bit. Bound by HBM: 4NK bytes read; U loads in flight
+// per lane (one at a time the 6912 x 2560 matrix took 23-25 us, with 20 12.4: 5.7 TB/s). U is the
+// smallest that holds a row of up to 1280: twenty for short ones read and added the last element over
+// and over (20000 x 64 8.7 us, one at a time 3.7).
+template <int U>
 __global__ __launch_bounds__(kBlock) void k_row_absmean(const float* __restrict__ W, size_t N,
                                                         size_t K, float inv_k, float* __restrict__ tau)
 {
@@ -53,7 +56,6 @@ __global__ __launch_bounds__(kBlock) void k_row_absmean(const float* __restrict_
     const size_t row = (size_t)blockIdx.x * (kBlock / kWave) + (threadIdx.x >> 6);
     if (row >= N) return;
     const float* w = W + row * K;
-    constexpr int U = 20;
     float acc = 0.0f;
     for (size_t k0 = (size_t)lane; k0 < K; k0 += U * kWave)
     {
@@ -336,7 +338,14 @@ hipError_t launch_row_absmean(hipStream_t st, const float* W, size_t N, size_t K
     if (N == 0) return hipSuccess;
     const float inv_k = 1.0f / (float)K;
     const unsigned grid = (unsigned)ceil_div(N, kBlock / kWave);
-    hipLaunchKernelGGL(k_row_absmean, dim3(grid), dim3(kBlock), 0, st, W, N, K, inv_k, tau);
+    const size_t loads = ceil_div(K, kWave);  // of a lane
+    const auto kern = loads <= 1    ? k_row_absmean<1>
+                      : loads <= 2  ? k_row_absmean<2>
+                      : loads <= 5  ? k_row_absmean<5>
+                      : loads <= 10 ? k_row_absmean<10>
+                      : loads <= 16 ? k_row_absmean<16>
+                                    : k_row_absmean<20>;
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), 0, st, W, N, K, inv_k, tau);
     return hipGetLastError();
 }
 

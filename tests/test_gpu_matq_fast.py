@@ -462,3 +462,39 @@ def test_matmul_f_special_token_time(ctx, N, K, M):
         return min(t)
 
     assert best(X2) <= 15.0 * best(X)
+
+
+@pytest.mark.parametrize("N,K", [(5, 1), (300, 64), (31, 65), (7, 127), (33, 129), (64, 320), (65, 321), (9, 640), (9, 641), (6, 1024),
+                                 (6, 1025), (5, 1280)])
+def test_absmean_short_rows(ctx, orc, N, K):
+    """The number of loads in flight per lane follows the row length (1, 2, 5, 10, 16 or 20 x 64 columns): each
+    one's ends, exact."""
+    W = normal((N, K), 11 * N + K, 0.0, 0.02)
+    W[N // 2, K // 2] = -0.0
+    assert np.array_equal(ctx.row_absmean(dev(W)).cpu().numpy(), orc.row_absmean(W))
+
+
+def test_absmean_short_row_time(ctx):
+    """Rows of 64 take no more than 0.7 of the time of rows of 512 (0.5 here; with twenty loads per lane for
+    both it was 0.95)."""
+    import torch
+
+    def best(K):
+        W = torch.randn((20000, K), device="cuda")
+        e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        g = torch.cuda.CUDAGraph()
+        ctx.row_absmean(W)
+        torch.cuda.synchronize()
+        with torch.cuda.graph(g):
+            for _ in range(20):
+                ctx.row_absmean(W)
+        t = []
+        for _ in range(8):
+            e[0].record()
+            g.replay()
+            e[1].record()
+            e[1].synchronize()
+            t.append(e[0].elapsed_time(e[1]))
+        return min(t)
+
+    assert best(64) <= 0.7 * best(512)
