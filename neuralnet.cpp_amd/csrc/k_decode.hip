@@ -840,12 +840,14 @@ hipError_t launch_copy_cols(hipStream_t st, const float* src, size_t rows, size_
 hipError_t launch_embed(hipStream_t st, const float* table, const int32_t* ids, size_t V, size_t d, size_t B, bool tm,
                         float* out)
 {
-    // below a tile of tokens the scattered stores are few (48 tokens 3.0 against 3.3 us, 64 3.3 both,
-    // 128 4.4 against 3.4)
-    if (!tm && B >= kEmbTile && ceil_div(d, kEmbTile) <= 65535)  // (grid limit)
+    // Few tiles leave most CUs idle and a block's round trip through LDS alone on the clock, while the
+    // scattered stores are few (element per thread / tiles, us: 300 x 64 tokens, 5 tiles 2.3 / 3.0,
+    // 1024 x 128, 32 tiles 2.7 / 3.1, 300 x 512, 40 tiles 3.6 / 3.2, 2560 x 64, 40 tiles 3.1 both,
+    // 2560 x 128, 80 tiles 4.3 / 3.2)
+    const size_t tb = ceil_div(B, kEmbTile), tf = ceil_div(d, kEmbTile);
+    if (!tm && B >= kEmbTile && tb * tf >= 40 && tf <= 65535)  // (grid limit)
     {
-        k_embed_cols<<<dim3((unsigned)ceil_div(B, kEmbTile), (unsigned)ceil_div(d, kEmbTile)), kSmallBlock, 0, st>>>(
-            table, ids, (int)V, (int)d, (int)B, out);
+        k_embed_cols<<<dim3((unsigned)tb, (unsigned)tf), kSmallBlock, 0, st>>>(table, ids, (int)V, (int)d, (int)B, out);
         return hipGetLastError();
     }
     k_embed<<<dim3((unsigned)ceil_div(d, kSmallBlock), (unsigned)B), kSmallBlock, 0, st>>>(table, ids, (int)V, (int)d,
