@@ -298,7 +298,8 @@ nnhip_status nnhip_ternary_matmul(nnhip_ctx* ctx, const void* rp, const float* t
  * combined in int64; results match a float64 evaluation far inside the reference tolerance
  * (1e-4 x max(1, max|Y|)). A token holding NaN or an infinity gets the IEEE result of its
  * non-finite terms per row (NaN for NaN, 0 x inf or opposite infinities, else the infinity).
- * K < 131072. Uses context scratch (grown on demand).
+ * K < 131072, and the digit rows, 4 * round_up(K, 256) * M bytes, below 4 GiB (from K = 65281 on the
+ * digit products too, 16 * N * M bytes). Uses context scratch (grown on demand).
  * Replaces ComputeEngine::matmul_q on the BitLinear f32 branch (include/neuralnet.cpp/
  * compute_layer_bitlinear.hpp:459-466; src/ternary_gemm_test.cpp:253-289) when the weights are
  * kept repacked; nnhip_matmul_q takes the reference container. */

@@ -895,6 +895,8 @@ static nnhip_status matmul_digits(nnhip_ctx* ctx, const char* fn, const void* rp
     NNHIP_REQUIRE(rp && B && Y, fn, "null pointer");
     NNHIP_REQUIRE(aligned16(rp), fn, "rp must be 16-byte aligned");
     NNHIP_REQUIRE(M <= kMaxDim / 4 && mul_ok(N, 4 * M), fn, "size overflow");
+    // four digit rows per token, behind the same 32-bit buffer ranges as the activations
+    NNHIP_REQUIRE(4 * round_up(K, kTileK) * M <= 0xFFFFFFFFull, fn, "the activations' digit rows must be below 4 GiB");
     // the digit products are exact integers in f32 while 128 K < 2^24
     if (K >= 131072) return fail(NNHIP_ERR_UNSUPPORTED, fn, "K must be below 131072 (use nnhip_matmul_q)");
     if (digit_gemv_ok(N, K, M, b_f16 != 0, B))
@@ -960,6 +962,8 @@ static nnhip_status matmul_digits(nnhip_ctx* ctx, const char* fn, const void* rp
         NNHIP_LAUNCH(fn, launch_gemm_digits(ctx->stream, p, out, ctx->num_cus, ctx->gemm_tile));
         return NNHIP_OK;
     }
+    // the digit products in f32, whose tail stores are sent to offset 0xFFFFFFF0
+    NNHIP_REQUIRE(N * M4 * 4 <= 0xFFFFFFF0ull, fn, "the digit products (K above 65280) must be below 4 GiB");
     const size_t b_yp = round_up(N * M4 * 4, 256), b_part = digit_part_bytes(M);
     st = ensure_ws(ctx, b_xi + b_rs + b_ex + b_yp + b_part, fn);
     if (st != NNHIP_OK) return st;

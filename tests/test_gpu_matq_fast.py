@@ -498,3 +498,29 @@ def test_absmean_short_row_time(ctx):
         return min(t)
 
     assert best(64) <= 0.7 * best(512)
+
+
+def test_matmul_f_token_limit(ctx, nnhip):
+    """The digit rows of the activations stay below 4 GiB, which the kernels address with 32 bits: the last
+    token count under that is exact in every token (K = 1: tau x trit x x), the next is refused before
+    anything is allocated or launched; likewise the digit products of K > 65280."""
+    import torch
+    M = (1 << 22) - 1
+    say(f"ternary_matmul_f token limit M={M}")
+    W = torch.tensor([[0.5], [-0.25], [0.0]], device="cuda")
+    tau = ctx.row_absmean(W)
+    rp = ctx.repack(ctx.trit_pack(W, tau), 1)
+    X = torch.randn((1, M + 1), device="cuda")
+    Y = ctx.ternary_matmul_f(rp, tau, X[:, :M].contiguous(), 3, 1)
+    assert torch.equal(Y[:2], torch.cat([0.5 * X[:, :M], -0.25 * X[:, :M]])) and not bool(Y[2].any())
+    with pytest.raises(nnhip.NNHipError) as e:
+        ctx.ternary_matmul_f(rp, tau, X, 3, 1)
+    assert e.value.status == 1
+    # K > 65280 (buffers of their full size: a size that is not refused is a valid call)
+    N, K, M = 16400, 65281, 16383
+    assert 4 * nnhip.kp(K) * M < 1 << 32 < 16 * N * M
+    rp = torch.zeros(nnhip.repacked_bytes(N, K) // 4, device="cuda", dtype=torch.int32)
+    X = torch.empty((K, M), device="cuda", dtype=torch.float16)
+    with pytest.raises(nnhip.NNHipError) as e:
+        ctx.ternary_matmul_f(rp, torch.ones(N, device="cuda"), X, N, K, out_f16=True)
+    assert e.value.status == 1
