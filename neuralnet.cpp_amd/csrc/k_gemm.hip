@@ -588,7 +588,7 @@ struct Gemm
     // 32-row block for j = 0..3.
     struct DigOps
     {
-        int nrs[kTB];      // -2 rowsum of the lane's digit rows, shifted as the sums are
+        uint32_t nrs[kTB]; // -2 rowsum of the lane's digit rows, shifted as the sums are
         int ex[kTB];       // the tokens' exponents
         float tv[kRBf][4]; // tau of the lane's output rows
     };
@@ -603,7 +603,7 @@ struct Gemm
         for (int n = 0; n < kTB; ++n)
         {
             const uint32_t m = (uint32_t)(4 * (t0 + n) + c);
-            e.nrs[n] = -(2 * __builtin_bit_cast(int, __builtin_amdgcn_raw_buffer_load_b32(rrs, m * 4u, 0, 0))) * (1 << (8 * (c & 1)));
+            e.nrs[n] = (0u - 2u * __builtin_amdgcn_raw_buffer_load_b32(rrs, m * 4u, 0, 0)) << (8 * (c & 1));
             e.ex[n] = __builtin_bit_cast(int, __builtin_amdgcn_raw_buffer_load_b32(rex, (uint32_t)(t0 + n) * 4u, 0, 0));
         }
 #pragma unroll
@@ -619,8 +619,8 @@ struct Gemm
 
     // T = sum_p A_p 256^p per (row, token) over the lane quad, then y = tau * (fl(T) * 2^(E - 30)).
     // Lane c holds A_c of rows 0..3 (of each group of four) and ends with row c: the xor-1 step adds
-    // A_0 + 256 A_1 or A_2 + 256 A_3 (below 2^31 while K <= 65280), the xor-2 step brings the other
-    // half. H 2^16 + L is exact in f64, so its conversion is the one rounding of fl(T). Special
+    // A_0 + 256 A_1 or A_2 + 256 A_3 (within int32 while K <= 65280; the shifted sums of codes on the way
+    // there are not, so they are added modulo 2^32), the xor-2 step brings the other half. H 2^16 + L is exact in f64, so its conversion is the one rounding of fl(T). Special
     // tokens (k_digits.hip has written their rows) and tokens past M are not stored.
     static __device__ __forceinline__ void store_dig(const GemvProblem& p, const DigitOut& g, const v16i (&acc)[kRB][kTB],
                                                      const DigOps& e, int rb0, int nrb, int row_w, int t0, int h, int c)
@@ -648,13 +648,13 @@ struct Gemm
 #pragma unroll
                 for (int n = 0; n < kTB; ++n)
                 {
-                    int a[4];
+                    uint32_t a[4];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) a[i] = (acc[rb][n][4 * j + i] << sh) + e.nrs[n];
+                    for (int i = 0; i < 4; ++i) a[i] = ((uint32_t)acc[rb][n][4 * j + i] << sh) + e.nrs[n];
                     // quad_perm [1,0,3,2] and [2,3,0,1]
-                    const int u = (odd ? a[1] : a[0]) + __builtin_amdgcn_mov_dpp(odd ? a[0] : a[1], 0xB1, 0xF, 0xF, true);
-                    const int v = (odd ? a[3] : a[2]) + __builtin_amdgcn_mov_dpp(odd ? a[2] : a[3], 0xB1, 0xF, 0xF, true);
-                    const int keep = high ? v : u, recv = __builtin_amdgcn_mov_dpp(high ? u : v, 0x4E, 0xF, 0xF, true);
+                    const uint32_t u = (odd ? a[1] : a[0]) + (uint32_t)__builtin_amdgcn_mov_dpp((int)(odd ? a[0] : a[1]), 0xB1, 0xF, 0xF, true);
+                    const uint32_t v = (odd ? a[3] : a[2]) + (uint32_t)__builtin_amdgcn_mov_dpp((int)(odd ? a[2] : a[3]), 0xB1, 0xF, 0xF, true);
+                    const int keep = (int)(high ? v : u), recv = __builtin_amdgcn_mov_dpp((int)(high ? u : v), 0x4E, 0xF, 0xF, true);
                     const double T = __builtin_fma((double)keep, s_keep, (double)recv * s_recv);
                     y[n] = e.tv[r][j] * __builtin_ldexpf((float)T, e.ex[n] - 30);
                 }

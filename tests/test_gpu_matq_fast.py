@@ -524,3 +524,28 @@ def test_matmul_f_token_limit(ctx, nnhip):
     with pytest.raises(nnhip.NNHipError) as e:
         ctx.ternary_matmul_f(rp, torch.ones(N, device="cuda"), X, N, K, out_f16=True)
     assert e.value.status == 1
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+@pytest.mark.parametrize("K", [65280, 65281])
+def test_matmul_f_longest_fused_digits(ctx, orc, K, tile):
+    """The longest reduction whose digit sums the GEMM's epilogue combines (K = 65280) and the first past it,
+    with the automatic choice and each tile: the digits at their ends (-128, 127 and 128 x 255 patterns) times
+    +1 and -1 in every column, so the sums are as large as they get, bit for bit."""
+    N, M = 40, 9
+    say(f"ternary_matmul_f longest fused digits K={K} tile={tile}")
+    W = np.full((N, K), 0.02, np.float32)
+    W[1::2] = -0.02
+    W[2::4, 1::2] *= -1.0
+    wq, tau, rp = case(ctx, orc, N, K, W=W)
+    assert np.all(np.abs(orc.trits_of(wq, K)) == 1)
+    X = np.empty((K, M), np.float32)
+    for m, d in enumerate([-0x808080, 0x7F7F7F, 0x808080, -0x7F7F7F, 0x7F807F, -0x80, 0x7F, 0xFFFFFF, -0xFFFFFF]):
+        X[:, m] = np.float32(d * 2.0 ** -30)
+        X[0, m] = 0.75                                   # E = 0: x 2^30 is the fixed point
+    ctx.set_gemm_tile(tile)
+    try:
+        got = host(ctx.ternary_matmul_f(rp, dev(tau), dev(X), N, K))
+    finally:
+        ctx.set_gemm_tile(0)
+    assert same_bits(got, digit_model(orc.trits_of(wq, K), X, tau=tau))
