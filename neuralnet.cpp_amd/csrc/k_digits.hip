@@ -836,11 +836,13 @@ hipError_t launch_digits(hipStream_t st, const void* B, bool b16, const float* k
                          int32_t* rowsum, int32_t* ex, uint32_t* part, const DigitSpecials& sp)
 {
     const size_t Kp = round_up(K, kTileK);
-    // one launch, one block per token, while the column reads stay few: there a lone call of the two
-    // launches takes 1-2 us longer (whole product before the fused combine, one against two launches:
-    // K=2560 M=40 23.4 / 24.6 us, M=256 44.5 / 42.1; K=1000 M=256 15.5 / 16.6; K=6912 M=5 26.0 /
-    // 28.1, M=8 29.4 / 28.3)
-    if (M <= 6 || (K <= 4096 && K * M <= (size_t(1) << 18)))
+    // one launch, one block per token, while there is a block for each CU at most and their column reads
+    // stay few: there the second launch costs 1-2 us more than the reads (whole product of 640 rows, one /
+    // two launches, us: K=256 M=256 8.0 / 10.0, 400 11.5 / 10.9, 1000 18.5 / 12.9; K=1000 M=200 11.7 /
+    // 12.9; K=2560 M=40 11.4 / 12.3, 100 13.0 / 13.4, 200 18.3 / 16.7; K=4096 M=64 14.7 / 15.1, 128
+    // 20.6 / 18.2; K=6912 M=12 14.0 / 15.6, 16 16.6 / 16.5, 40 18.7 / 17.2; K=11008 M=12 19.0 / 19.9,
+    // 24 23.9 / 22.0)
+    if (M <= 6 || (M <= 256 && K * M <= (K <= 4096 ? size_t(1) << 18 : size_t(1) << 17)))
     {
         k_digits<<<dim3((unsigned)M), kDigThreads, 0, st>>>(B, b16, kscale, (int)K, (int)M, (int)Kp, xi, rowsum, ex, sp);
         return hipGetLastError();

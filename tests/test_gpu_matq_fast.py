@@ -500,6 +500,20 @@ def test_absmean_short_row_time(ctx):
     assert best(64) <= 0.7 * best(512)
 
 
+@pytest.mark.parametrize("N,K,M", [(33, 5000, 26), (33, 5000, 27), (20, 256, 256), (20, 256, 257), (20, 2560, 102),
+                                   (20, 2560, 103), (20, 11008, 7)])
+def test_matmul_f_digit_launches(ctx, orc, N, K, M):
+    """Either side of the line between one block per token and blocks of 64 tokens, bit for bit the digit
+    model."""
+    say(f"ternary_matmul_f digit launches N={N} K={K} M={M}")
+    wq, tau, rp = case(ctx, orc, N, K, seed=N + K + M)
+    X = normal((K, M), 60 + M)
+    X[:, ::3] *= 17.0
+    X[K - 1, M - 1] = 99.0
+    got = host(ctx.ternary_matmul_f(rp, dev(tau), dev(X), N, K))
+    assert same_bits(got, digit_model(orc.trits_of(wq, K), X, tau=tau))
+
+
 def test_matmul_f_token_limit(ctx, nnhip):
     """The digit rows of the activations stay below 4 GiB, which the kernels address with 32 bits: the last
     token count under that is exact in every token (K = 1: tau x trit x x), the next is refused before
