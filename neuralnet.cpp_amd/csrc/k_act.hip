@@ -8,7 +8,7 @@
 // are bit-identical to the unfused reference sequence whichever kernel runs.
 //
 // Kernels by shape:
-//   k_token_regs   M > 64, K up to 512 * 22: 8 tokens per 16-wave block (mostly M > 1024 and
+//   k_token_regs   M > 64, K up to 512 * 22: 8 tokens per 16-wave block (M > 1024 and
 //                  K <= 7168), else 4 per 8-wave block. Each
 //                  thread loads its rows (16 B = 4 tokens per row) once and keeps them in
 //                  registers through the passes (sum of squares, absmax, quantize), so X is read
@@ -884,11 +884,13 @@ static hipError_t launch_token_kernel(hipStream_t st, const float* X, const floa
         // just written, K = 2560, M = 512 9.4 against 11.0 us, K = 6912, M = 1024 17.4 against 20.2)
         // and a thread's rows fit the 128 registers of a 1024-thread block (K <= 7168). Measured the
         // same way, 8 against 4 tokens: 2560 x 8192 27.8 / 34.5 us, 2560 x 32768 138 / 169, 4096 x 8192
-        // 48 / 59, 6912 x 8192 90 / 96; with RMSNorm past 10 rounds 6912 x 4096 43.8 / 42.4 and
-        // 6912 x 3333 (rows off the 16-byte grid) 40.0 / 45.4, so those take 8 from M = 4096 or M % 4.
+        // 48 / 59; with RMSNorm past 10 rounds, at one block to a CU, 5200 x 2048 18.4 / 19.5, 5632 x 1500
+        // 16.9 / 20.5, 6144 x 3333 33.6 / 38.6, 6912 x 4096 38.0 / 41.1, 7168 x 16384 196 / 212 (a few
+        // tokens past whole rounds of blocks the smaller ones finish sooner: 5632 x 4100 42.6 / 38.1,
+        // 7168 x 4100 53.2 / 52.1).
         TokArgs a{X, norm, eps, inv_f, (int)K, (int)M, (int)Kp, mode, xi, s, rowsum, xq_ref, fout};
         const bool plain = !norm && mode == 0;
-        const bool tok8 = M > 1024 && rounds <= 14 && (plain || rounds <= 10 || M > 4096 || M % 4 != 0);
+        const bool tok8 = M > 1024 && rounds <= 14;
         // One resident round of 8-token blocks (M <= 2048) writes the codes through the L2 as they are
         // produced: 4096 x 2048 13.9 -> 12.6 us. More rounds don't: right after X was written it cost
         // 4096 x 8192 48 -> 69 us, 6912 x 8192 86 -> 129.

@@ -238,6 +238,20 @@ def test_token_blocks_edges(ctx, orc, F, M, shift):
     assert np.array_equal(host(ctx.rmsnorm(Xd, dev(g), 1e-6)), orc.rmsnorm(X, g, 1e-6))
 
 
+@pytest.mark.parametrize("F,M", [(5121, 1028), (5632, 2048), (7168, 1100), (6912, 4096)])
+def test_token_blocks_wide_rows(ctx, orc, F, M):
+    """RMSNorm over 11 to 14 rounds of 512 features in 8-token blocks, whole quads of tokens: codes, scales
+    and sums exact."""
+    say(f"token blocks, wide rows F={F} M={M}")
+    X = normal((F, M), F + M, 0.0, 1.0)
+    g = normal((F,), 3, 1.0, 0.1)
+    xi, s, rs = ctx.rmsnorm_quant_i8(dev(X), dev(g), 1e-6)
+    xq_o, s_o = orc.rmsnorm_quant_i8(X, g, 1e-6)
+    q = orc.container_to_int8(xq_o, M).T
+    assert np.array_equal(host(s), s_o) and np.array_equal(host(xi)[:, :F], q) and np.all(host(xi)[:, F:] == 0)
+    assert np.array_equal(host(rs), q.astype(np.int64).sum(axis=1))
+
+
 @pytest.mark.parametrize("F,M,loc", [(2560, 33, 0.0), (6912, 64, 3.0), (1, 5, 0.0), (17, 1, -1.0), (300, 1000, 0.5),
                                      (13, 2048, 0.0), (2560, 31, 0.0)])
 def test_layernorm(ctx, orc, F, M, loc):
