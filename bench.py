@@ -33,7 +33,6 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0          # MI355X HBM3E
 INT8_PEAK_TOPS = 5000.0        # MI355X dense int8 MFMA (5.0 POP/s)
-FP32_MFMA_PEAK_TFLOPS = 157.3  # MI355X dense fp32 MFMA
 LAYERS = 30
 D, FFN, KV = 2560, 6912, 640
 SHAPES = [("q", D, D), ("k", D, KV), ("v", D, KV), ("o", D, D),
@@ -454,7 +453,6 @@ def _c5_measure(ctx, torch, stream, steps, nn, dm, dec, cfg, prompt, wbytes):
     res = {
         "prefill_ms": round(t_prefill * 1e3, 3), "prefill_tokens_per_s": round(B * ctx_len / t_prefill, 1),
         "prefill_attention_one_layer": {"us": round(t_pfa * 1e6, 1), "TFLOP/s": round(pfa_flops / t_pfa / 1e12, 1),
-                                        "frac_fp32_mfma": round(pfa_flops / t_pfa / 1e12 / FP32_MFMA_PEAK_TFLOPS, 4),
                                         "flops": pfa_flops},
         "tokens_per_s": round(B / t_step, 1), "ms_per_step": round(t_step * 1e3, 4),
         "eager_ms_per_step": round(t_eager * 1e3, 4),

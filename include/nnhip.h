@@ -598,9 +598,12 @@ nnhip_status nnhip_kv_cache_fill_h(nnhip_ctx* ctx, const float* k, const float* 
 /* Causal attention of the T tokens over caches already holding rows [0, pos0 + T) (after
  * nnhip_kv_cache_fill): out (H*dk, B*T), column b*T + t = per query head h the softmax
  * ((rot(q_h) . K^T) * scale) . V over cache rows [0, pos0 + t] of sequence b, KV head h / (H/Hkv),
- * q rotated at pos0 + t. f32 operands as two f16 halves on the f16 MFMA with an online softmax: within 2e-6 relative of a
- * float64 evaluation (the reference does not pin the order). dk in {64, 128}; H / Hkv in
- * {1, 2, 4, 8}. Replaces the attention steps of T AttentionBase::forward_step calls
+ * q rotated at pos0 + t. f32 operands as sums of f16 or bf16 parts on the MFMA, f32 sums and softmax
+ * (the reference does not pin the order): each output within 2e-6 of its sum of |probability x value|
+ * of a float64 evaluation for scores up to about 10 (N(0, 1) inputs), whatever the other values are;
+ * larger scores carry an f32 score's rounding, as f32 products do. Inputs that the parts cannot hold
+ * (non-finite ones, scores that could reach 2^18, outputs below 2^-100) take f32 products, up to 1.5
+ * times as long as those alone. dk in {64, 128}; H / Hkv in {1, 2, 4, 8}. Replaces the attention steps of T AttentionBase::forward_step calls
  * (compute_layer_attention.hpp:1022-1083). */
 nnhip_status nnhip_attention_prefill(nnhip_ctx* ctx, const float* q, const float* k_cache, const float* v_cache,
                                      size_t B, size_t T, size_t H, size_t Hkv, size_t dk, size_t pos0,

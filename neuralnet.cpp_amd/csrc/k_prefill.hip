@@ -61,17 +61,12 @@ namespace
 
 typedef float v16f __attribute__((ext_vector_type(16)));
 
-constexpr int kPQ = 32;   // queries per work-group
+constexpr int kPQ = 32;   // queries per wave of the attention, tokens per block of the cache fill
 constexpr int kPK = 32;   // keys per tile
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t pf_rsrc(const void* base, uint32_t bytes)
 {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
-}
-
-__device__ __forceinline__ float ld_f(__amdgpu_buffer_rsrc_t r, uint32_t off)
-{
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
 }
 
 __device__ __forceinline__ float4 ld_f4(__amdgpu_buffer_rsrc_t r, uint32_t off)

@@ -6,8 +6,8 @@ compute_layer_attention.hpp:1003-1091), then the whole prefill of Decoder.prefil
 
 The cache rows (rotated keys, values) are compared bit for bit. The attention output is compared
 within 5e-6 x max(1, max|out|) of the oracle: its dot products and softmax sums are f32 in an
-order the reference leaves open, and the prefill kernel sums f16-half products in f32 with an
-online softmax.
+order the reference leaves open, and the prefill kernel sums products of f16 and bf16 parts in f32
+with an online softmax.
 """
 import math
 
@@ -373,16 +373,16 @@ def attend64(q, kc, vc, B, T, H, Hkv, dk, pos0, scale):
     return out, mag
 
 
-# value scales of (q, keys, values): ordinary, powers of two far apart, ends of the f16 halves' range,
-# and past it (f32 products)
+# value scales of (q, keys, values): ordinary, powers of two far apart, ends of the range that the f16
+# halves take, and past it (f32 products)
 SCALES = [(1.0, 1.0, 1.0), (1e3, 1e-3, 1e-9), (1e-6, 1e6, 1e12), (1e-13, 1e13, 1.0), (1e20, 1e-20, 1e25), (1.0, 1.0, 1e-30)]
 
 
 @pytest.mark.parametrize("f16", [False, True])
 @pytest.mark.parametrize("H,Hkv,dk,T,pos0", [(4, 4, 64, 257, 3), (4, 2, 128, 129, 31), (8, 1, 64, 33, 64), (4, 1, 128, 65, 0)])
 def test_prefill_halves_match_float64(ctx, H, Hkv, dk, T, pos0, f16):
-    """The f16-halves products at every group size, tails of queries and keys, values whose scale
-    rises and falls along the sequence, scores that keep growing, and scales past the halves' range:
+    """The products in parts at every group size, tails of queries and keys, values whose scale
+    rises and falls along the sequence, scores that keep growing, and scales past the parts' range:
     within 1e-5 of float64 relative to sum |p v| (f32 scores of magnitude up to 25: 25 x 2^-24 each
     in the exponent, and sums of at most 321 keys)."""
     import torch
