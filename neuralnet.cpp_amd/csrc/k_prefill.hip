@@ -721,7 +721,7 @@ __global__ __launch_bounds__(kPThreads) void k_attn_prefill(PrefillArgs a)
         }
         if (w.live && kb * kPK <= a.pos0 + w.t0 + kPQ - 1)
         {
-            // S^T = K . Q^T: the products of the halves but low x low (2^-24 of a term)
+            // S^T = K . Q^T: the products of the halves but low x low (at most 2^-22 of a term)
             v16f s = v16f{};
 #pragma unroll
             for (int g = 0; g < GKN; ++g)
